@@ -9,125 +9,14 @@
 //   window tiles, sink blocks and routed blocks in one softmax state; the
 //   split entry points below run the window and the rest as two launches
 //   merged by LSE).
-// f32: attn_f32_kernel, one thread per (query, head), sequential fp32 dot
-//   products and a two-pass softmax; the fp32 parity path.
+// f32: hba_attn_f32.hip (fp32 MFMA; the fp32 parity path).
 #include "hba_common.h"
 #include "hba_abi.h"
 #include "hba_generic.h"
 #include "hba_attn_bf16.h"
-
-namespace hba {
-
-// ------------------------------------------------------------ fp32 path ----
-template <int D>
-__device__ __forceinline__ float dot_row(const float (&qv)[D], const float *k) {
-    float a = 0.0f;
-#pragma unroll
-    for (int t = 0; t < D; t += 4) {
-        float4 kv = *reinterpret_cast<const float4 *>(k + t);
-        a = fmaf(qv[t], kv.x, a);
-        a = fmaf(qv[t + 1], kv.y, a);
-        a = fmaf(qv[t + 2], kv.z, a);
-        a = fmaf(qv[t + 3], kv.w, a);
-    }
-    return a;
-}
-
-template <int D>
-__global__ __launch_bounds__(64) void attn_f32_kernel(
-    const float *__restrict__ q, int64_t qsb, int64_t qsn, int64_t qsh, const float *__restrict__ qgain,
-    float eps, const float *__restrict__ kc, const float *__restrict__ kr, const float *__restrict__ vt,
-    const float *__restrict__ cosT, const float *__restrict__ sinT, const int32_t *__restrict__ idx,
-    const int32_t *__restrict__ cnt, int64_t n, int Hq, int Hkv, int S, int64_t W, int kk, float scale,
-    float *__restrict__ out, int64_t osb, int64_t osn, int64_t osh) {
-    const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
-    const int h = blockIdx.y;
-    const int64_t b = blockIdx.z;
-    if (i >= n) return;
-    const int G = Hq / Hkv;
-    const int g = h / G;
-    float qc[D], qr[D];
-    const float *qrow = q + b * qsb + i * qsn + (int64_t)h * qsh;
-#pragma unroll
-    for (int t = 0; t < D; t += 4) {
-        float4 u = *reinterpret_cast<const float4 *>(qrow + t);
-        qc[t] = u.x;
-        qc[t + 1] = u.y;
-        qc[t + 2] = u.z;
-        qc[t + 3] = u.w;
-    }
-    if (qgain) qknorm_row<0, D>(qc, qgain[h], eps);
-    rope_row<0, D>(qc, qr, cosT + i * D, sinT + i * D);
-    const int64_t bh = b * Hkv + g;
-    const float *KC = kc + bh * n * D;
-    const float *KR = kr + bh * n * D;
-    const float *VT = vt + bh * D * n;
-    const int64_t s_end = ((int64_t)S < i + 1) ? (int64_t)S : i + 1;
-    const int64_t w_beg = ((int64_t)S > i - W + 1) ? (int64_t)S : i - W + 1;
-    const int c = min(max(cnt[bh * n + i], 0), kk);
-    const int32_t *ix = idx + (bh * n + i) * kk;
-    const int64_t nb = n / 64;
-    float mx = -INFINITY;
-    for (int64_t j = 0; j < s_end; ++j) mx = fmaxf(mx, dot_row<D>(qc, KC + j * D) * scale);
-    for (int64_t j = w_beg; j <= i; ++j) mx = fmaxf(mx, dot_row<D>(qr, KR + j * D) * scale);
-    // a routed block's keys below S are sinks, counted once (the union mask
-    // of attention.py:351-352; with S <= 64 no routed block holds one)
-    for (int r = 0; r < c; ++r) {
-        if (ix[r] < 1 || ix[r] >= nb) continue;   // block 0 is never routed (sinks, window)
-        const int64_t j0 = (int64_t)ix[r] * 64;
-        for (int64_t j = (j0 > S ? j0 : S); j < j0 + 64; ++j) mx = fmaxf(mx, dot_row<D>(qc, KC + j * D) * scale);
-    }
-    float acc[D];
-#pragma unroll
-    for (int t = 0; t < D; ++t) acc[t] = 0.0f;
-    float l = 0.0f;
-    for (int64_t j = 0; j < s_end; ++j) {
-        float p = expf(dot_row<D>(qc, KC + j * D) * scale - mx);
-        l += p;
-#pragma unroll
-        for (int t = 0; t < D; ++t) acc[t] = fmaf(p, VT[(int64_t)t * n + j], acc[t]);
-    }
-    for (int64_t j = w_beg; j <= i; ++j) {
-        float p = expf(dot_row<D>(qr, KR + j * D) * scale - mx);
-        l += p;
-#pragma unroll
-        for (int t = 0; t < D; ++t) acc[t] = fmaf(p, VT[(int64_t)t * n + j], acc[t]);
-    }
-    for (int r = 0; r < c; ++r) {
-        if (ix[r] < 1 || ix[r] >= nb) continue;   // block 0 is never routed (sinks, window)
-        const int64_t j0 = (int64_t)ix[r] * 64;
-        for (int64_t j = (j0 > S ? j0 : S); j < j0 + 64; ++j) {
-            float p = expf(dot_row<D>(qc, KC + j * D) * scale - mx);
-            l += p;
-#pragma unroll
-            for (int t = 0; t < D; ++t) acc[t] = fmaf(p, VT[(int64_t)t * n + j], acc[t]);
-        }
-    }
-    float *orow = out + b * osb + i * osn + (int64_t)h * osh;
-    float inv = 1.0f / l;
-#pragma unroll
-    for (int t = 0; t < D; ++t) orow[t] = acc[t] * inv;
-}
-
-}  // namespace hba
+#include "hba_attn_f32.h"
 
 using namespace hba;
-
-namespace {
-template <int D>
-int launch_attn_f32(const void *q, const int64_t *qs, const float *qgain, float eps, const void *kc,
-                    const void *kr, const void *vt, const float *cosT, const float *sinT,
-                    const int32_t *idx, const int32_t *cnt, int64_t B, int64_t n, int64_t Hq,
-                    int64_t Hkv, int64_t S, int64_t W, int64_t k, float scale, void *out,
-                    const int64_t *os, hipStream_t s) {
-    dim3 grid((unsigned)((n + 63) / 64), (unsigned)Hq, (unsigned)B);
-    hipLaunchKernelGGL(attn_f32_kernel<D>, grid, dim3(64), 0, s, (const float *)q, qs[0], qs[1], qs[2],
-                       qgain, eps, (const float *)kc, (const float *)kr, (const float *)vt, cosT, sinT,
-                       idx, cnt, n, (int)Hq, (int)Hkv, (int)S, W, (int)k, scale, (float *)out, os[0],
-                       os[1], os[2]);
-    return HBA_OK;
-}
-}  // namespace
 
 extern "C" int hba_attn_fwd_workspace_bytes(int dtype, int64_t B, int64_t n, int64_t Hq, int64_t d,
                                             size_t *bytes) {

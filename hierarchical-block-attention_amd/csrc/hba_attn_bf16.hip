@@ -37,6 +37,7 @@
 #include "hba_abi.h"
 #include "hba_attn_bf16.h"
 #include "hba_dma.h"
+#include "hba_xcd.h"
 
 namespace hba {
 namespace ab {
@@ -203,26 +204,6 @@ __device__ __forceinline__ void qoperand(const bf16_t *q, int64_t qsb, int64_t q
         qpack_rope<D>(x, cosT, sinT, i, valid, lg, qscale, qop);
     else
         qpack<D>(x, valid, qscale, qop);
-}
-
-// Workgroup -> (batch*KV head combo, query tile).  Workgroup i runs on XCD
-// i % 8; xmap 1 (8 % Cn == 0) and 2 (Cn % 8 == 0) give each XCD one combo's
-// keys at a time, so the blocks it gathers share that XCD's L2.  Tiles go
-// deepest first: a tile's union of routed blocks grows with its candidate
-// count, and starting the longest workgroups first leaves the short ones to
-// fill the end.
-__device__ __forceinline__ void xcd_map(int i, int Cn, int ntiles, int xmap, int &combo, int &tile) {
-    if (xmap == 1) {
-        combo = (i & 7) % Cn;
-        tile = (i >> 3) * (8 / Cn) + (i & 7) / Cn;
-    } else if (xmap == 2) {
-        combo = (i / (8 * ntiles)) * 8 + (i & 7);
-        tile = (i >> 3) % ntiles;
-    } else {
-        combo = i / ntiles;
-        tile = i % ntiles;
-    }
-    if (tile < ntiles) tile = ntiles - 1 - tile;   // padding workgroups (xmap 1) keep tile >= ntiles
 }
 
 // ======================================================== tile staging ====
@@ -1690,19 +1671,6 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void bwd_dq_union_kernel(
 }
 
 // ============================================================ launchers ====
-static void grid_map(int64_t Cn, int64_t ntiles, int &xmap, int64_t &grid) {
-    if (8 % Cn == 0) {
-        xmap = 1;   // 8 workgroups per round, 8/Cn tiles of each combo per round
-        grid = 8 * ((ntiles + (8 / Cn) - 1) / (8 / Cn));
-    } else if (Cn % 8 == 0) {
-        xmap = 2;
-        grid = Cn * ntiles;
-    } else {
-        xmap = 0;
-        grid = Cn * ntiles;
-    }
-}
-
 template <int D, int RT>
 static int launch_win(const void *q, const int64_t *qs, const float *qgain, const float *kgain, float eps,
                       const void *kr, const void *vt, const float *cosT, const float *sinT, int64_t B, int64_t n,
@@ -1756,9 +1724,8 @@ static int launch_routed_t(const void *q, const int64_t *qs, const float *qgain,
     const size_t lds = routed_lds<D, PTW>(n, G, k);
     const int64_t QT = (int64_t)C::WAVES * PTW * (16 / G);
     const int64_t ntiles = (n + QT - 1) / QT;
-    int xmap;
     int64_t grid;
-    grid_map(B * Hkv, ntiles, xmap, grid);
+    const int xmap = xcd_pick(B * Hkv, ntiles, grid);
     if (grid > 0x7fffffff) return HBA_ERR_UNSUPPORTED;
     const int Wc = (int)((W < n + 1) ? W : n + 1);     // a window longer than the sequence is the sequence
     auto go = [&](auto kern) -> int {
@@ -1813,9 +1780,8 @@ static int launch_dq_t(const void *q, const float *qgain, const float *kgain, fl
     const size_t lds = dq_lds<D, WAVES, PTW, NS>(n, G, k);
     const int64_t QT = (int64_t)WAVES * PTW * (16 / G);
     const int64_t ntiles = (n + QT - 1) / QT;
-    int xmap;
     int64_t grid;
-    grid_map(B * Hkv, ntiles, xmap, grid);
+    const int xmap = xcd_pick(B * Hkv, ntiles, grid);
     if (grid > 0x7fffffff) return HBA_ERR_UNSUPPORTED;
     const int Wc = (int)((W < n + 1) ? W : n + 1);     // a window longer than the sequence is the sequence
     auto kern = &bwd_dq_union_kernel<D, WAVES, PTW, NS, PH>;

@@ -1,0 +1,17 @@
+// Launchers of the fp32 union attention on the fp32 matrix cores: the forward
+// (launch_attn_f32; any query heads per KV head, sinks, k and window) and the
+// backward's query and key gradients (G <= 16, S <= 64, k <= 64).
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace hba {
+
+template <int D>
+int launch_attn_f32(const void *q, const int64_t *qs, const float *qgain, float eps, const void *kc, const void *kr,
+                    const void *vt, const float *cosT, const float *sinT, const int32_t *idx, const int32_t *cnt,
+                    int64_t B, int64_t n, int64_t Hq, int64_t Hkv, int64_t S, int64_t W, int64_t k, float scale,
+                    void *out, const int64_t *os, hipStream_t s);
+
+}  // namespace hba
