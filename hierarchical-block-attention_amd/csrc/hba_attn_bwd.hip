@@ -18,29 +18,21 @@
 // fp32 throughout; storage roundings of the forward are treated as identity,
 // as autograd treats the reference's casts.
 //
-// fp32 inputs take two VALU kernels:
-//   bwd_dq:  one wave per (b, i, KV head g), lanes over d, the G heads of the
-//            group in registers.  Pass 1 recomputes the union LSE, pass 2
-//            accumulates dq; it also leaves the QKNorm'd and rotated query
-//            rows, the LSE and D in the workspace for bwd_dkv.
-//   bwd_dkv: one workgroup per (b, g, 64-key block); a lane holds 16 elements
-//            of one key (keys x 16-element chunks per wave) and walks the
-//            query rows that attend its keys: the window rows, the sink rows
-//            (block 0), and the rows whose selection holds the block (found by
-//            scanning the selection lists into LDS).
+// fp32 inputs take the kernels of hba_attn_f32_bwd.hip (fp32 matrix cores).
 // bf16 inputs take the same gradients on MFMA: bwd_kt (transposed keys),
 // bwd_dq_mfma (16/G queries per wave, their heads the columns of 16-wide
 // tiles, one online pass), bwd_dkv_mfma (64 (row, head) pairs per tile, one
 // workgroup per key block and row range)
 // and bwd_dkv_fin (rope^T and the QKNorm backward of the key rows); a second
-// bwd_dkv_mfma launch takes the sink keys.  The fp32 path takes the sink keys
-// in bwd_sink.  Both split the sink keys' query rows over workgroups.
+// bwd_dkv_mfma launch takes the sink keys, their query rows split over
+// workgroups.
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
 
 #include "hba_abi.h"
 #include "hba_attn_bf16.h"
+#include "hba_attn_f32.h"
 #include "hba_generic.h"
 #include "hba_common.h"
 
@@ -79,211 +71,8 @@ __device__ __forceinline__ float wsum(float v) {
     return (a + b) + (c + d);
 }
 
-// element e of lane l is t = l + 64 e; GM = the largest group size held
-template <int DT, int D, int GM>
-__global__ __launch_bounds__(256) void bwd_dq_kernel(
-    const typename St<DT>::T *__restrict__ q, const typename St<DT>::T *__restrict__ kc,
-    const typename St<DT>::T *__restrict__ kr, const typename St<DT>::T *__restrict__ v,
-    const float *__restrict__ qgain, float eps, const float *__restrict__ cosT, const float *__restrict__ sinT,
-    const int32_t *__restrict__ idx, const int32_t *__restrict__ cnt, const typename St<DT>::T *__restrict__ out,
-    const typename St<DT>::T *__restrict__ dout, int B, int64_t n, int Hq, int Hkv, int S, int64_t W, int kk,
-    float scale, float *__restrict__ qc_ws, float *__restrict__ qr_ws, float *__restrict__ lse_ws,
-    float *__restrict__ dd_ws, float *__restrict__ sink_acc, typename St<DT>::T *__restrict__ dq,
-    float *__restrict__ dq_gain) {
-    constexpr int E = D / 64;
-    const int lane = threadIdx.x & 63;
-    const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (wid >= (int64_t)B * Hkv * n) return;                      // wave-uniform
-    const int64_t i = wid % n;
-    const int g = (int)((wid / n) % Hkv);
-    const int b = (int)(wid / (n * Hkv));
-    const int G = Hq / Hkv;
-    const int64_t nb = n / 64;
-    if (i < 64) {   // clear key row i of the sink accumulators (bwd_sink adds into them next)
-        float *acc = sink_acc + (((int64_t)b * Hkv + g) * 2 * 64 + i) * D;
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            acc[lane + 64 * e] = 0.0f;
-            acc[64 * D + lane + 64 * e] = 0.0f;
-        }
-    }
-
-    float xr[GM][E], qcv[GM][E], qrv[GM][E], dov[GM][E];
-    float rr[GM], msr[GM], dd[GM];
-    float cs[E], sn[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int t = lane + 64 * e;
-        cs[e] = St<DT>::rnd(cosT[i * D + t]);
-        sn[e] = St<DT>::rnd(sinT[i * D + t]);
-    }
-#pragma unroll
-    for (int hh = 0; hh < GM; ++hh) {
-        if (hh >= G) break;
-        const int h = g * G + hh;
-        const int64_t row = (((int64_t)b * n + i) * Hq + h) * D;
-        float ss = 0.0f, od = 0.0f;
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const int t = lane + 64 * e;
-            xr[hh][e] = St<DT>::ld(q, row + t);
-            dov[hh][e] = St<DT>::ld(dout, row + t);
-            ss = fmaf(xr[hh][e], xr[hh][e], ss);
-            od = fmaf(dov[hh][e], St<DT>::ld(out, row + t), od);
-        }
-        dd[hh] = wsum<D>(od);
-        msr[hh] = wsum<D>(ss) / (float)D;
-        const float r = sqrtf(fmaxf(msr[hh], eps));
-        rr[hh] = r;
-#pragma unroll
-        for (int e = 0; e < E; ++e)
-            qcv[hh][e] = qgain ? St<DT>::rnd((xr[hh][e] / r) * qgain[h]) : xr[hh][e];
-        // rotation: the partner of element t is t ^ (D/2)
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const int t = lane + 64 * e;
-            const float pv = (D == 64) ? __shfl_xor(qcv[hh][0], 32, 64) : qcv[hh][e ^ 1];
-            const float rot = (t < D / 2) ? -pv : pv;
-            qrv[hh][e] = St<DT>::rnd(St<DT>::rnd(qcv[hh][e] * cs[e]) + St<DT>::rnd(rot * sn[e]));
-            qc_ws[row + t] = qcv[hh][e];
-            qr_ws[row + t] = qrv[hh][e];
-        }
-    }
-    const int64_t bg = (int64_t)b * Hkv + g;
-    const int64_t wlo = (S > i - W + 1) ? (int64_t)S : i - W + 1;   // window [wlo, i]
-    const int64_t nsink = ((int64_t)S < i + 1) ? (int64_t)S : i + 1;
-    const int ncnt = min(max(cnt[bg * n + i], 0), kk);
-    const int32_t *sel = idx + (bg * n + i) * kk;
-    // the keys of the union in a fixed order: sinks, window, routed picks
-    const int64_t nwin = (i >= wlo) ? i - wlo + 1 : 0;                 // empty for i < S
-    const int64_t nkeys = nsink + nwin + (int64_t)ncnt * 64;
-    auto key_of = [&](int64_t u, bool &rope, bool &ok) -> int64_t {
-        rope = false;
-        ok = true;
-        if (u < nsink) return u;
-        u -= nsink;
-        if (u < nwin) {
-            rope = true;
-            return wlo + u;
-        }
-        u -= nwin;
-        const int blk = sel[u >> 6];
-        ok = blk >= 1 && (int64_t)blk < nb;
-        return ok ? 64 * (int64_t)blk + (u & 63) : 0;
-    };
-    const typename St<DT>::T *KC = kc + bg * n * D, *KR = kr + bg * n * D;
-
-    // pass 1: the union LSE of each head
-    float m[GM], l[GM];
-#pragma unroll
-    for (int hh = 0; hh < GM; ++hh) {
-        m[hh] = -INFINITY;
-        l[hh] = 0.0f;
-    }
-    for (int64_t u = 0; u < nkeys; ++u) {
-        bool rope, ok;
-        const int64_t j = key_of(u, rope, ok);
-        if (!ok) continue;
-        float kv[E];
-#pragma unroll
-        for (int e = 0; e < E; ++e) kv[e] = St<DT>::ld(rope ? KR : KC, j * D + lane + 64 * e);
-#pragma unroll
-        for (int hh = 0; hh < GM; ++hh) {
-            if (hh >= G) break;
-            float pr = 0.0f;
-#pragma unroll
-            for (int e = 0; e < E; ++e) pr = fmaf(rope ? qrv[hh][e] : qcv[hh][e], kv[e], pr);
-            const float s = wsum<D>(pr) * scale;
-            const float mn = fmaxf(m[hh], s);
-            l[hh] = l[hh] * __expf(m[hh] - mn) + __expf(s - mn);
-            m[hh] = mn;
-        }
-    }
-    float lse[GM];
-#pragma unroll
-    for (int hh = 0; hh < GM; ++hh) {
-        if (hh >= G) break;
-        lse[hh] = (l[hh] > 0.0f) ? m[hh] + __logf(l[hh]) : INFINITY;   // no key: every p is 0
-        if (lane == 0) {
-            const int64_t o = ((int64_t)b * Hq + g * G + hh) * n + i;
-            lse_ws[o] = lse[hh];
-            dd_ws[o] = dd[hh];
-        }
-    }
-
-    // pass 2: dq (NoPE and rotated parts)
-    float gc[GM][E], gr[GM][E];
-#pragma unroll
-    for (int hh = 0; hh < GM; ++hh)
-#pragma unroll
-        for (int e = 0; e < E; ++e) gc[hh][e] = gr[hh][e] = 0.0f;
-    const typename St<DT>::T *V = v + ((int64_t)b * n * Hkv + g) * D;   // v[b, j, g, :] at j * Hkv * D
-    for (int64_t u = 0; u < nkeys; ++u) {
-        bool rope, ok;
-        const int64_t j = key_of(u, rope, ok);
-        if (!ok) continue;
-        float kv[E], vv[E];
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            kv[e] = St<DT>::ld(rope ? KR : KC, j * D + lane + 64 * e);
-            vv[e] = St<DT>::ld(V, j * Hkv * D + lane + 64 * e);
-        }
-#pragma unroll
-        for (int hh = 0; hh < GM; ++hh) {
-            if (hh >= G) break;
-            float pr = 0.0f, pd = 0.0f;
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                pr = fmaf(rope ? qrv[hh][e] : qcv[hh][e], kv[e], pr);
-                pd = fmaf(dov[hh][e], vv[e], pd);
-            }
-            const float s = wsum<D>(pr) * scale;
-            const float dp = wsum<D>(pd);
-            const float p = __expf(s - lse[hh]);
-            const float ds = p * (dp - dd[hh]) * scale;
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                if (rope) gr[hh][e] = fmaf(ds, kv[e], gr[hh][e]);
-                else gc[hh][e] = fmaf(ds, kv[e], gc[hh][e]);
-            }
-        }
-    }
-
-    // rope^T, then the QKNorm backward, per head
-#pragma unroll
-    for (int hh = 0; hh < GM; ++hh) {
-        if (hh >= G) break;
-        const int h = g * G + hh;
-        const int64_t row = (((int64_t)b * n + i) * Hq + h) * D;
-        float y[E], zs[E];
-#pragma unroll
-        for (int e = 0; e < E; ++e) zs[e] = gr[hh][e] * sn[e];
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const int t = lane + 64 * e;
-            const float pv = (D == 64) ? __shfl_xor(zs[0], 32, 64) : zs[e ^ 1];
-            y[e] = gc[hh][e] + gr[hh][e] * cs[e] + ((t < D / 2) ? pv : -pv);
-        }
-        if (qgain) {
-            const float gn = qgain[h];
-            const float r = rr[hh];
-            float yx = 0.0f;
-#pragma unroll
-            for (int e = 0; e < E; ++e) yx = fmaf(y[e], xr[hh][e], yx);
-            yx = wsum<D>(yx);
-            const float corr = (msr[hh] >= eps) ? gn * yx / ((float)D * r * r * r) : 0.0f;
-#pragma unroll
-            for (int e = 0; e < E; ++e) y[e] = (gn / r) * y[e] - xr[hh][e] * corr;
-            if (lane == 0 && dq_gain) atomicAdd(&dq_gain[h], yx / r);
-        }
-#pragma unroll
-        for (int e = 0; e < E; ++e) St<DT>::st(dq, row + lane + 64 * e, y[e]);
-    }
-}
-
 // -------------------------------------------------- bwd_dq on MFMA (bf16) ----
-// The same gradient as bwd_dq_kernel with every product on
-// v_mfma_f32_16x16x32_bf16.  A wave takes qpw = 16 / G consecutive queries
+// The query gradient with every product on v_mfma_f32_16x16x32_bf16.  A wave takes qpw = 16 / G consecutive queries
 // (at most 4) of one (b, g); the 16 tile columns are its (query, head) pairs
 // (l16 = column).  The keys come in 64-key units (the sink unit, the window
 // pages, the routed blocks):
@@ -386,7 +175,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dq_mfma_kernel(
     const int32_t *__restrict__ idx, const int32_t *__restrict__ cnt, const bf16_t *__restrict__ out,
     const bf16_t *__restrict__ dout, int B, int64_t n, int Hq, int Hkv, int S, int64_t W, int kk, float scale,
     int qpw, bf16_t *__restrict__ qc_ws, bf16_t *__restrict__ qr_ws, float *__restrict__ lse_ws,
-    float *__restrict__ dd_ws, float *__restrict__ sink_acc, bf16_t *__restrict__ dq, float *__restrict__ dq_gain) {
+    float *__restrict__ dd_ws, bf16_t *__restrict__ dq, float *__restrict__ dq_gain) {
     constexpr int NKS = D / 32, NDT = D / 16, E = D / 64;
     // the window pages of the workgroup's queries, staged once for its four
     // waves: K and V rows [64][D + 8], K^T rows [D][64 + 8]
@@ -406,16 +195,6 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dq_mfma_kernel(
     const int b = (int)(blockIdx.x / (nwg * Hkv));
     const int64_t nb = n / 64;
     const int64_t bg = (int64_t)b * Hkv + g;
-    for (int qq = 0; act && qq < qpw; ++qq) {   // clear key row i of the sink accumulators (bwd_sink adds into them next)
-        const int64_t ic = i0 + qq;
-        if (ic >= 64 || ic >= n) break;
-        float *acc = sink_acc + (bg * 2 * 64 + ic) * D;
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            acc[lane + 64 * e] = 0.0f;
-            acc[64 * D + lane + 64 * e] = 0.0f;
-        }
-    }
     // column l16 = (query qs of the wave, head l16 - qs G)
     const int qs = l16 / G;
     const int64_t iq = i0 + qs;
@@ -726,238 +505,6 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dq_mfma_kernel(
     }
 }
 
-// ------------------------------------------------------------- bwd_dkv ----
-// Lane (kl, c) = (lane / NC, lane % NC) of wave w: key j = 64 blk + KW w + kl,
-// elements 16c .. 16c+15; a key's chunks sit on NC adjacent lanes, so its
-// sums are DPP steps within a quad (NC = 4) or an 8-lane group (NC = 8).
-template <int D>
-struct DkvCfg {
-    static constexpr int NC = D / 16;          // 16-element chunks per key
-    static constexpr int KW = 64 / NC;         // keys per wave
-    static constexpr int WAVES = 64 / KW;      // waves per 64-key block
-    static constexpr int NT = WAVES * 64;
-};
-
-template <int D>
-__device__ __forceinline__ float chunk_sum(float v) {
-    if constexpr (DkvCfg<D>::NC == 4) return quad_sum(v);
-    else return oct_sum(v);
-}
-
-template <int DT>
-__device__ __forceinline__ void ld16(const typename St<DT>::T *p, float (&x)[16]) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) x[e] = St<DT>::ld(p, e);
-}
-
-// nrows query rows (row_of(r)), all G heads of KV head g, against this lane's
-// key j: accumulates gk += ds * x (x = the stored query rows qx_ws: NoPE or
-// rotated) and gv += p * dO.  mode 0: window rows (j >= S, j <= i <= j+W-1),
-// 1: sink rows (j < S, i >= j), 2: routed rows (every key of the block).  The
-// next row's operands are loaded while the current one is computed.
-template <int DT, int D, typename RowOf>
-__device__ __forceinline__ void dkv_rows(RowOf row_of, int64_t nrows, int mode, int64_t j, int S, int64_t W,
-                                         const float *qx_ws, const typename St<DT>::T *dout,
-                                         const float *lse_ws, const float *dd_ws, int b, int64_t n, int Hq,
-                                         int g, int G, int c, float scale, const float (&ky)[16],
-                                         const float (&vv)[16], float (&gk)[16], float (&gv)[16]) {
-    const int64_t total = nrows * G;
-    if (total <= 0) return;
-    auto load = [&](int64_t u, float (&x)[16], float (&dv)[16], float &lse, float &dd, int64_t &i) {
-        i = row_of(u / G);
-        const int h = g * G + (int)(u % G);
-        const int64_t ro = (((int64_t)b * n + i) * Hq + h) * D + 16 * c;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) x[e] = qx_ws[ro + e];
-        ld16<DT>(dout + ro, dv);
-        const int64_t so = ((int64_t)b * Hq + h) * n + i;
-        lse = lse_ws[so];
-        dd = dd_ws[so];
-    };
-    auto compute = [&](const float (&x)[16], const float (&dov)[16], float lse, float dd, int64_t i) {
-        const bool valid = (mode == 0) ? (j >= S && i >= j && i <= j + W - 1) : (mode == 1) ? (j < S && i >= j)
-                                                                                           : true;
-        float pr = 0.0f, pd = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            pr = fmaf(x[e], ky[e], pr);
-            pd = fmaf(dov[e], vv[e], pd);
-        }
-        const float sc = chunk_sum<D>(pr) * scale;
-        const float dp = chunk_sum<D>(pd);
-        const float p = valid ? __expf(sc - lse) : 0.0f;
-        const float ds = p * (dp - dd) * scale;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            gv[e] = fmaf(p, dov[e], gv[e]);
-            gk[e] = fmaf(ds, x[e], gk[e]);
-        }
-    };
-    float xa[16], da[16], xb[16], db[16], la, ldd, lb, ldb;
-    int64_t ia, ib;
-    load(0, xa, da, la, ldd, ia);
-    for (int64_t u = 0; u < total; u += 2) {
-        if (u + 1 < total) load(u + 1, xb, db, lb, ldb, ib);
-        compute(xa, da, la, ldd, ia);
-        if (u + 1 >= total) break;
-        if (u + 2 < total) load(u + 2, xa, da, la, ldd, ia);
-        compute(xb, db, lb, ldb, ib);
-    }
-}
-
-// Sink keys (block 0, j < S) against query rows [r0, r0 + SINK_ROWS): one
-// workgroup per (b, g, row range), the lanes laid out as in bwd_dkv; the
-// partial gradients are added (fp32 atomics) into sink_acc [B, Hkv, 2, 64, D]
-// (dk then dv), which bwd_dkv's block-0 workgroup reads.
-constexpr int SINK_ROWS = 256;
-
-template <int DT, int D>
-__global__ __launch_bounds__(DkvCfg<D>::NT) void bwd_sink_kernel(
-    const typename St<DT>::T *__restrict__ kc, const typename St<DT>::T *__restrict__ v,
-    const typename St<DT>::T *__restrict__ dout, int64_t n, int Hq, int Hkv, int S, int nsplit, float scale,
-    const float *__restrict__ qc_ws, const float *__restrict__ lse_ws, const float *__restrict__ dd_ws,
-    float *__restrict__ sink_acc) {
-    using C = DkvCfg<D>;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int kl = lane / C::NC, c = lane % C::NC;
-    const int split = (int)(blockIdx.x % nsplit);
-    const int g = (int)((blockIdx.x / nsplit) % Hkv);
-    const int b = (int)(blockIdx.x / ((int64_t)nsplit * Hkv));
-    const int G = Hq / Hkv;
-    if (C::KW * w >= S) return;                                   // wave-uniform; no barrier follows
-    const int64_t j = C::KW * w + kl;
-    const int64_t bg = (int64_t)b * Hkv + g;
-    float kcv[16], vv[16], gkc[16], gv[16];
-    ld16<DT>(kc + (bg * n + j) * D + 16 * c, kcv);
-    ld16<DT>(v + (((int64_t)b * n + j) * Hkv + g) * D + 16 * c, vv);
-#pragma unroll
-    for (int e = 0; e < 16; ++e) gkc[e] = gv[e] = 0.0f;
-    const int64_t r0 = (int64_t)split * SINK_ROWS;
-    const int64_t r1 = min(n, r0 + SINK_ROWS);
-    dkv_rows<DT, D>([&](int64_t r) { return r0 + r; }, r1 - r0, 1, j, S, 0, qc_ws, dout, lse_ws, dd_ws, b, n, Hq, g,
-                    G, c, scale, kcv, vv, gkc, gv);
-    if (j < S) {
-        float *acc = sink_acc + (bg * 2 * 64 + j) * D + 16 * c;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            atomicAdd(acc + e, gkc[e]);
-            atomicAdd(acc + 64 * D + e, gv[e]);
-        }
-    }
-}
-
-template <int DT, int D>
-__global__ __launch_bounds__(DkvCfg<D>::NT) void bwd_dkv_kernel(
-    const typename St<DT>::T *__restrict__ k, const typename St<DT>::T *__restrict__ kc,
-    const typename St<DT>::T *__restrict__ kr, const typename St<DT>::T *__restrict__ v,
-    const float *__restrict__ kgain, float eps, const float *__restrict__ cosT, const float *__restrict__ sinT,
-    const int32_t *__restrict__ idx, const int32_t *__restrict__ cnt, const typename St<DT>::T *__restrict__ dout,
-    int64_t n, int Hq, int Hkv, int S, int64_t W, int kk, float scale, const float *__restrict__ qc_ws,
-    const float *__restrict__ qr_ws, const float *__restrict__ lse_ws, const float *__restrict__ dd_ws,
-    const float *__restrict__ sink_acc, typename St<DT>::T *__restrict__ dk, typename St<DT>::T *__restrict__ dv,
-    float *__restrict__ dk_gain) {
-    using C = DkvCfg<D>;
-    __shared__ int rows[C::NT];
-    __shared__ int wcount[C::WAVES];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int kl = lane / C::NC, c = lane % C::NC;
-    const int64_t nb = n / 64;
-    const int blk = (int)(blockIdx.x % nb);
-    const int g = (int)((blockIdx.x / nb) % Hkv);
-    const int b = (int)(blockIdx.x / (nb * Hkv));
-    const int G = Hq / Hkv;
-    const int64_t j = 64 * (int64_t)blk + C::KW * w + kl;       // this lane's key
-    const int64_t bg = (int64_t)b * Hkv + g;
-    const int64_t kro = (bg * n + j) * D + 16 * c;              // kc / kr row chunk
-    const int64_t rro = (((int64_t)b * n + j) * Hkv + g) * D + 16 * c;   // k / v / dk / dv row chunk
-    float kcv[16], krv[16], vv[16], gkc[16], gkr[16], gv[16];
-    ld16<DT>(kc + kro, kcv);
-    ld16<DT>(kr + kro, krv);
-    ld16<DT>(v + rro, vv);
-#pragma unroll
-    for (int e = 0; e < 16; ++e) gkc[e] = gkr[e] = gv[e] = 0.0f;
-
-    // window rows (rotated): key j >= S is in the window of queries j .. j + W - 1
-    {
-        const int64_t j0 = 64 * (int64_t)blk + C::KW * w;           // the wave's first key
-        const int64_t ihi = min(n - 1, j0 + C::KW - 1 + W - 1);
-        dkv_rows<DT, D>([&](int64_t r) { return j0 + r; }, ihi - j0 + 1, 0, j, S, W, qr_ws, dout, lse_ws, dd_ws, b,
-                        n, Hq, g, G, c, scale, krv, vv, gkr, gv);
-    }
-    // sink keys (NoPE): every query i >= j; their rows were split over the
-    // bwd_sink workgroups, whose sums are added here
-    if (blk == 0 && j < S) {
-        const float *acc = sink_acc + (bg * 2 * 64 + j) * D + 16 * c;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            gkc[e] += acc[e];
-            gv[e] += acc[64 * D + e];
-        }
-    }
-    // routed rows (NoPE): the queries whose selection holds this block
-    if (blk >= 1) {
-        for (int64_t i0 = 0; i0 < n; i0 += C::NT) {
-            const int64_t i = i0 + tid;
-            bool picked = false;
-            if (i < n) {
-                const int nc = min(max(cnt[bg * n + i], 0), kk);
-                const int32_t *sl = idx + (bg * n + i) * kk;
-                for (int r = 0; r < nc; ++r) picked |= sl[r] == blk;
-            }
-            const uint64_t bal = __ballot(picked);
-            if (lane == 0) wcount[w] = __popcll(bal);
-            __syncthreads();
-            int base = 0, tot = 0;
-            for (int u = 0; u < C::WAVES; ++u) {
-                if (u < w) base += wcount[u];
-                tot += wcount[u];
-            }
-            if (picked) rows[base + __popcll(bal & ((1ull << lane) - 1ull))] = (int)i;
-            __syncthreads();
-            dkv_rows<DT, D>([&](int64_t r) { return (int64_t)rows[r]; }, tot, 2, j, S, W, qc_ws, dout, lse_ws, dd_ws,
-                            b, n, Hq, g, G, c, scale, kcv, vv, gkc, gv);
-            __syncthreads();                                     // rows[] and wcount[] reused
-        }
-    }
-
-    // rope^T at position j, then the QKNorm backward of k row (b, j, g)
-    float y[16];
-    {
-        float zs[16];
-        const float *cp = cosT + j * D + 16 * c, *sp = sinT + j * D + 16 * c;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) zs[e] = gkr[e] * St<DT>::rnd(sp[e]);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const float pv = __shfl_xor(zs[e], C::NC / 2, 64);      // chunk c ^ (NC/2): element t ^ (D/2)
-            y[e] = gkc[e] + gkr[e] * St<DT>::rnd(cp[e]) + ((c < C::NC / 2) ? pv : -pv);
-        }
-    }
-    if (kgain) {
-        float x[16];
-        ld16<DT>(k + rro, x);
-        float ss = 0.0f, yx = 0.0f;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            ss = fmaf(x[e], x[e], ss);
-            yx = fmaf(y[e], x[e], yx);
-        }
-        const float ms = chunk_sum<D>(ss) / (float)D;
-        yx = chunk_sum<D>(yx);
-        const float r = sqrtf(fmaxf(ms, eps));
-        const float gn = kgain[g];
-        const float corr = (ms >= eps) ? gn * yx / ((float)D * r * r * r) : 0.0f;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) y[e] = (gn / r) * y[e] - x[e] * corr;
-        if (c == 0 && dk_gain) atomicAdd(&dk_gain[g], yx / r);
-    }
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        St<DT>::st(dk, rro + e, y[e]);
-        St<DT>::st(dv, rro + e, gv[e]);
-    }
-}
-
 // ------------------------------------------------ bwd_dkv on MFMA (bf16) ----
 // dK and dV of one 64-key block from the (query row, head) pairs that attend
 // it, 64 pairs per tile staged in LDS twice (row-major and transposed), taken
@@ -982,6 +529,7 @@ __global__ __launch_bounds__(DkvCfg<D>::NT) void bwd_dkv_kernel(
 // per (b, g, range of sink_rows rows) against block 0, every row of the range
 // attending the keys j < S with j <= i (NoPE); waves whose 16 keys hold no
 // sink skip the products.
+constexpr int SINK_ROWS = 256;   // query rows per workgroup of the sink launch
 constexpr int DKV_RL = 1024;   // routed rows run as one series of tiles at most
 constexpr int DKV_TP = 64;   // pairs per tile: two halves of 32, the pair count of one product
 
@@ -1258,7 +806,7 @@ __global__ __launch_bounds__(DKV_NT, D == 64 ? 4 : 2) void bwd_dkv_mfma_kernel(
 
 // dk / dv of key rows (b, j, g), lane = element d (and d + 64); a wave takes
 // FIN_RPW consecutive rows, a workgroup one 64-key block: the summed NoPE /
-// rotated dk and dv (plus the sink accumulators for j < S), rope^T at
+// rotated dk and dv, rope^T at
 // position j, then the QKNorm backward of k row (b, j, g).  The gain gradient
 // is summed over the workgroup's 64 rows before its one atomic add (the adds
 // of all workgroups meet on Hkv addresses).
@@ -1266,9 +814,8 @@ constexpr int FIN_RPW = 16;
 template <int D>
 __global__ __launch_bounds__(256) void bwd_dkv_fin_kernel(
     const bf16_t *__restrict__ k, const float *__restrict__ kgain, float eps, const float *__restrict__ cosT,
-    const float *__restrict__ sinT, int64_t n, int Hkv, int S, const float *__restrict__ dkv_acc,
-    const float *__restrict__ sink_acc, bf16_t *__restrict__ dk, bf16_t *__restrict__ dv,
-    float *__restrict__ dk_gain) {
+    const float *__restrict__ sinT, int64_t n, int Hkv, const float *__restrict__ dkv_acc,
+    bf16_t *__restrict__ dk, bf16_t *__restrict__ dv, float *__restrict__ dk_gain) {
     constexpr int E = D / 64;
     __shared__ float gsum[4];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -1286,11 +833,6 @@ __global__ __launch_bounds__(256) void bwd_dkv_fin_kernel(
             gkc[e] = a[d];
             gkr[e] = a[D + d];
             gv[e] = a[2 * D + d];
-            if (j < S && sink_acc) {
-                const float *sa = sink_acc + (bg * 2 * 64 + j) * D;
-                gkc[e] += sa[d];
-                gv[e] += sa[64 * D + d];
-            }
             zs[e] = gkr[e] * rnd_bf16(sinT[j * D + d]);
         }
         float y[E];
@@ -1346,8 +888,8 @@ static bool bwd_dq_union_on() {
 }
 
 // Workspace of hba_attn_bwd: the query rows in the storage type (QKNorm'd,
-// rotated), LSE and D per (head, row), the fp32 sink accumulators
-// [B, Hkv, 2, 64, d]; on the bf16 path also the transposed keys kct, krt
+// rotated), LSE and D per (head, row), an unused [B, Hkv, 2, 64, d] fp32 (the
+// sizes are part of the ABI); on the bf16 path also the transposed keys kct, krt
 // [B, Hkv, d, n] and the fp32 dk / dv accumulators [B, Hkv, n, 3, d].
 namespace {
 struct BwdWs {
@@ -1438,20 +980,25 @@ extern "C" int hba_attn_bwd(int dtype, const void *q, const void *k, const void 
     const BwdWs L = bwd_ws_layout(dtype, B, n, Hq, Hkv, d);
     if (ws_bytes < L.total || !abi::aligned16(workspace)) return HBA_ERR_INVALID_ARG;
     char *wsb = (char *)workspace;
-    float *qc_ws = (float *)(wsb + L.qc);                          // fp32 path's query rows
-    float *qr_ws = (float *)(wsb + L.qr);
     bf16_t *qcb_ws = (bf16_t *)(wsb + L.qc);                       // bf16 path's query rows
     bf16_t *qrb_ws = (bf16_t *)(wsb + L.qr);
     float *lse_ws = (float *)(wsb + L.lse);
     float *dd_ws = (float *)(wsb + L.dd);
-    float *sink_acc = (float *)(wsb + L.sink);                     // [B, Hkv, 2, 64, d]
     bf16_t *kct = (bf16_t *)(wsb + L.kct);                         // [B, Hkv, d, n] (bf16 path)
     bf16_t *krt = (bf16_t *)(wsb + L.krt);
     float *dkv_acc = (float *)(wsb + L.dkv);                       // [B, Hkv, n, 3, d] (bf16 path)
     uint32_t *pbits = (uint32_t *)(wsb + L.pbits);                 // routed-row bits (bf16 path)
     hipStream_t s = (hipStream_t)stream;
-    const int64_t nwaves = B * Hkv * n;
-    const int64_t g1 = (nwaves + 3) / 4;
+    if (dtype == HBA_DTYPE_F32) {
+        const auto bwd = d == 64 ? launch_attn_bwd_f32<64> : launch_attn_bwd_f32<128>;
+        st = bwd((const float *)q, (const float *)k, (const float *)v, (const float *)kc, (const float *)kr, q_gain,
+                 k_gain, eps, cos_tab, sin_tab, idx, cnt, (const float *)out, (const float *)dout, B, n, Hq, Hkv, S, W,
+                 k_blocks, scale, (float *)(wsb + L.qc), (float *)(wsb + L.qr), lse_ws, dd_ws, (float *)dq, (float *)dk,
+                 (float *)dv, dq_gain, dk_gain, s);
+        if (st) return st;
+        HBA_LAUNCH_CHECK();
+        return HBA_OK;
+    }
     const int64_t g2 = B * Hkv * (n / 64);
     const int nsplit = (int)((n + bw::SINK_ROWS - 1) / bw::SINK_ROWS);
     const int64_t gs = B * Hkv * nsplit;
@@ -1466,67 +1013,43 @@ extern "C" int hba_attn_bwd(int dtype, const void *q, const void *k, const void 
     const int64_t gpb = (B * Hkv * n * k_blocks + 255) / 256;     // bwd_pick_bits: a thread per pick
     if (gpb > 0x7fffffffLL) return HBA_ERR_UNSUPPORTED;
     if (g3 > 0x7fffffffLL) return HBA_ERR_UNSUPPORTED;
-#define HBA_BWD(DT, D)                                                                                          \
+#define HBA_BWD(D)                                                                                              \
     do {                                                                                                        \
-        using T = St<DT>::T;                                                                                    \
-        if constexpr (DT == 1) {                                                                                \
-            hipLaunchKernelGGL((bw::bwd_kt_kernel<D>), dim3((unsigned)g2), dim3(256), 0, s, (const bf16_t *)kc,  \
-                               (const bf16_t *)kr, kct, krt, n, dkv_acc, pbits, nsplit_kv);                      \
-            hipLaunchKernelGGL(bw::bwd_pick_bits_kernel, dim3((unsigned)gpb), dim3(256), 0, s, idx, cnt, n,      \
-                               n / 64, (int)k_blocks, B * Hkv * n * k_blocks, nsplit_kv, pbits);                 \
-            int dqs = HBA_ERR_UNSUPPORTED;                                                                      \
-            if constexpr (D == 64)                                                                              \
-                if (bwd_dq_union_on())                                                                              \
-                    dqs = launch_attn_bf16_dq<D>(q, q_gain, k_gain, eps, kc, kr, kct, krt, v, cos_tab, sin_tab,  \
-                                                 idx, cnt, out, dout, B, n, Hq, Hkv, S, W, k_blocks, scale,      \
-                                                 qcb_ws, qrb_ws, lse_ws, dd_ws, dq, dq_gain, s);                 \
-            if (dqs == HBA_ERR_UNSUPPORTED)                                                                     \
-                hipLaunchKernelGGL((bw::bwd_dq_mfma_kernel<D>), dim3((unsigned)g1q), dim3(256), 0, s,            \
-                                   (const bf16_t *)q, (const bf16_t *)kc, (const bf16_t *)kr, kct, krt,         \
-                                   (const bf16_t *)v, q_gain, eps, cos_tab, sin_tab, idx, cnt,                  \
-                                   (const bf16_t *)out, (const bf16_t *)dout, (int)B, n, (int)Hq, (int)Hkv,     \
-                                   (int)S, W, (int)k_blocks, scale, qpw, qcb_ws, qrb_ws, lse_ws, dd_ws,         \
-                                   sink_acc, (bf16_t *)dq, dq_gain);                                            \
-            else if (dqs != HBA_OK)                                                                             \
-                return dqs;                                                                                     \
-        } else if (Hq / Hkv <= 8)                                                                               \
-            hipLaunchKernelGGL((bw::bwd_dq_kernel<DT, D, 8>), dim3((unsigned)g1), dim3(256), 0, s,               \
-                               (const T *)q, (const T *)kc, (const T *)kr, (const T *)v, q_gain, eps, cos_tab,   \
-                               sin_tab, idx, cnt, (const T *)out, (const T *)dout, (int)B, n, (int)Hq, (int)Hkv, \
-                               (int)S, W, (int)k_blocks, scale, qc_ws, qr_ws, lse_ws, dd_ws, sink_acc, (T *)dq,   \
-                               dq_gain);                                                                        \
-        else                                                                                                    \
-            hipLaunchKernelGGL((bw::bwd_dq_kernel<DT, D, bw::BW_GMAX>), dim3((unsigned)g1), dim3(256), 0, s,     \
-                               (const T *)q, (const T *)kc, (const T *)kr, (const T *)v, q_gain, eps, cos_tab,   \
-                               sin_tab, idx, cnt, (const T *)out, (const T *)dout, (int)B, n, (int)Hq, (int)Hkv, \
-                               (int)S, W, (int)k_blocks, scale, qc_ws, qr_ws, lse_ws, dd_ws, sink_acc, (T *)dq,   \
-                               dq_gain);                                                                        \
-        if (S > 0 && DT == 0)                                                                                   \
-            hipLaunchKernelGGL((bw::bwd_sink_kernel<DT, D>), dim3((unsigned)gs), dim3(bw::DkvCfg<D>::NT), 0, s,  \
-                               (const T *)kc, (const T *)v, (const T *)dout, n, (int)Hq, (int)Hkv, (int)S,       \
-                               nsplit, scale, qc_ws, lse_ws, dd_ws, sink_acc);                                   \
-        if constexpr (DT == 1) {                                                                                \
-            if (S > 0)                                                                                          \
-                hipLaunchKernelGGL((bw::bwd_dkv_mfma_kernel<D>), dim3((unsigned)gs), dim3(bw::DKV_NT), 0, s,     \
-                                   (const bf16_t *)kc, (const bf16_t *)kr, (const bf16_t *)v, idx, cnt,          \
-                                   (const bf16_t *)dout, n, (int)Hq, (int)Hkv, (int)S, W, (int)k_blocks, scale,  \
-                                   nsplit, qcb_ws, qrb_ws, lse_ws, dd_ws, cos_tab, sin_tab, pbits, dkv_acc,     \
-                                   bw::SINK_ROWS);                                                              \
-            hipLaunchKernelGGL((bw::bwd_dkv_mfma_kernel<D>), dim3((unsigned)g3), dim3(bw::DKV_NT), 0, s,         \
+        hipLaunchKernelGGL((bw::bwd_kt_kernel<D>), dim3((unsigned)g2), dim3(256), 0, s, (const bf16_t *)kc,      \
+                           (const bf16_t *)kr, kct, krt, n, dkv_acc, pbits, nsplit_kv);                          \
+        hipLaunchKernelGGL(bw::bwd_pick_bits_kernel, dim3((unsigned)gpb), dim3(256), 0, s, idx, cnt, n, n / 64,  \
+                           (int)k_blocks, B * Hkv * n * k_blocks, nsplit_kv, pbits);                             \
+        int dqs = HBA_ERR_UNSUPPORTED;                                                                          \
+        if constexpr (D == 64)                                                                                  \
+            if (bwd_dq_union_on())                                                                              \
+                dqs = launch_attn_bf16_dq<D>(q, q_gain, k_gain, eps, kc, kr, kct, krt, v, cos_tab, sin_tab,      \
+                                             idx, cnt, out, dout, B, n, Hq, Hkv, S, W, k_blocks, scale,          \
+                                             qcb_ws, qrb_ws, lse_ws, dd_ws, dq, dq_gain, s);                     \
+        if (dqs == HBA_ERR_UNSUPPORTED)                                                                         \
+            hipLaunchKernelGGL((bw::bwd_dq_mfma_kernel<D>), dim3((unsigned)g1q), dim3(256), 0, s,                \
+                               (const bf16_t *)q, (const bf16_t *)kc, (const bf16_t *)kr, kct, krt,             \
+                               (const bf16_t *)v, q_gain, eps, cos_tab, sin_tab, idx, cnt,                      \
+                               (const bf16_t *)out, (const bf16_t *)dout, (int)B, n, (int)Hq, (int)Hkv,         \
+                               (int)S, W, (int)k_blocks, scale, qpw, qcb_ws, qrb_ws, lse_ws, dd_ws,             \
+                               (bf16_t *)dq, dq_gain);                                                          \
+        else if (dqs != HBA_OK)                                                                                 \
+            return dqs;                                                                                         \
+        if (S > 0)                                                                                              \
+            hipLaunchKernelGGL((bw::bwd_dkv_mfma_kernel<D>), dim3((unsigned)gs), dim3(bw::DKV_NT), 0, s,         \
                                (const bf16_t *)kc, (const bf16_t *)kr, (const bf16_t *)v, idx, cnt,              \
                                (const bf16_t *)dout, n, (int)Hq, (int)Hkv, (int)S, W, (int)k_blocks, scale,      \
-                               nsplit_kv, qcb_ws, qrb_ws, lse_ws, dd_ws, cos_tab, sin_tab, pbits, dkv_acc, 0);   \
-            hipLaunchKernelGGL((bw::bwd_dkv_fin_kernel<D>), dim3((unsigned)g4), dim3(256), 0, s,                 \
-                               (const bf16_t *)k, k_gain, eps, cos_tab, sin_tab, n, (int)Hkv, (int)S, dkv_acc,    \
-                               (const float *)nullptr, (bf16_t *)dk, (bf16_t *)dv, dk_gain);                     \
-        } else                                                                                                  \
-            hipLaunchKernelGGL((bw::bwd_dkv_kernel<DT, D>), dim3((unsigned)g2), dim3(bw::DkvCfg<D>::NT), 0, s,   \
-                               (const T *)k, (const T *)kc, (const T *)kr, (const T *)v, k_gain, eps, cos_tab,   \
-                               sin_tab, idx, cnt, (const T *)dout, n, (int)Hq, (int)Hkv, (int)S, W,              \
-                               (int)k_blocks, scale, qc_ws, qr_ws, lse_ws, dd_ws, sink_acc, (T *)dk, (T *)dv,    \
-                               dk_gain);                                                                        \
+                               nsplit, qcb_ws, qrb_ws, lse_ws, dd_ws, cos_tab, sin_tab, pbits, dkv_acc,         \
+                               bw::SINK_ROWS);                                                                  \
+        hipLaunchKernelGGL((bw::bwd_dkv_mfma_kernel<D>), dim3((unsigned)g3), dim3(bw::DKV_NT), 0, s,             \
+                           (const bf16_t *)kc, (const bf16_t *)kr, (const bf16_t *)v, idx, cnt,                  \
+                           (const bf16_t *)dout, n, (int)Hq, (int)Hkv, (int)S, W, (int)k_blocks, scale,          \
+                           nsplit_kv, qcb_ws, qrb_ws, lse_ws, dd_ws, cos_tab, sin_tab, pbits, dkv_acc, 0);       \
+        hipLaunchKernelGGL((bw::bwd_dkv_fin_kernel<D>), dim3((unsigned)g4), dim3(256), 0, s,                     \
+                           (const bf16_t *)k, k_gain, eps, cos_tab, sin_tab, n, (int)Hkv, dkv_acc,               \
+                           (bf16_t *)dk, (bf16_t *)dv, dk_gain);                                                \
     } while (0)
-    HBA_DISPATCH_DT_D(dtype, d, HBA_BWD);
+    if (d == 64) HBA_BWD(64);
+    else HBA_BWD(128);
 #undef HBA_BWD
     HBA_LAUNCH_CHECK();
     return HBA_OK;

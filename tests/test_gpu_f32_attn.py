@@ -1,4 +1,4 @@
-"""The fp32 union attention (forward) at the edges of its tiles: group sizes
+"""The fp32 union attention (forward and backward) at the edges of its tiles: group sizes
 that fill, split and overflow a 16-column tile, pick lists of one and of
 several 64-pick chunks, repeated and invalid picks, sinks past the first
 block, windows of one key and of the whole sequence, and keys that are not
@@ -109,3 +109,105 @@ def test_keys_outside_the_union_are_not_read_into_it():
     clean = ~(inf | nan)
     ref = _reference(q, kc, kr, torch.nan_to_num(v, 0.0, 0.0, 0.0), gq, 1e-6, cos, sin, idx, cnt, S, W, scale)
     assert (out[:, clean].double() - ref[:, clean]).norm() <= 2e-6 * ref[:, clean].norm()
+
+
+def _norm_rope(x, gain, eps, cos, sin):
+    d = x.shape[-1]
+    x = x / x.pow(2).mean(-1, keepdim=True).clamp_min(eps).sqrt() * gain[:, None]
+    rot = torch.cat((-x[..., d // 2:], x[..., :d // 2]), -1)
+    return x, x * cos[:, None] + rot * sin[:, None]
+
+
+def _unique(idx, n):
+    """Repeated picks of a row become out-of-range ones."""
+    for t in range(1, idx.shape[-1]):
+        idx[..., t][(idx[..., :t] == idx[..., t:t + 1]).any(-1)] = n // 64
+    return idx
+
+
+def _grads(q, kx, v, gq, gk, idx, cnt, dout, S, W, scale, cos, sin):
+    """64-bit gradients of q, k, v and the gains."""
+    B, n, Hq, d = q.shape
+    G, nb = Hq // kx.shape[2], n // 64
+    leaf = [t.double().requires_grad_(True) for t in (q, kx, v, gq, gk)]
+    x, xr = _norm_rope(leaf[0], leaf[3], 1e-6, cos, sin)
+    y, yr = _norm_rope(leaf[1], leaf[4], 1e-6, cos, sin)
+    i, j = torch.arange(n)[:, None], torch.arange(n)[None, :]
+    sink, win = (j < S) & (j <= i), (j >= S) & (j <= i) & (j > i - W)
+    ok = (torch.arange(idx.shape[-1]) < cnt[..., None]) & (idx >= 1) & (idx < nb)
+    routed = torch.zeros(B, kx.shape[2], n, nb).scatter_add_(-1, idx.long().clamp(0, nb - 1), ok.float()) > 0
+    routed = routed.repeat_interleave(64, -1) & (j >= S)
+    total = 0.0
+    for b in range(B):
+        for h in range(Hq):
+            g = h // G
+            s = torch.cat((x[b, :, h] @ y[b, :, g].T, xr[b, :, h] @ yr[b, :, g].T), -1) * scale
+            # a key in the window and in a routed block counts in both frames
+            s = torch.cat((s, s[:, :n]), -1)
+            p = s.masked_fill(~torch.cat((sink, win, routed[b, g]), -1), -math.inf).softmax(-1)
+            o = (p[:, :n] + p[:, n:2 * n] + p[:, 2 * n:]) @ leaf[2][b, :, g]
+            total = total + (o * dout[b, :, h].double()).sum()
+    return torch.autograd.grad(total, leaf)
+
+
+def _run_bwd(q, kx, v, gq, gk, idx, cnt, dout, S, W):
+    dev = torch.device("cuda")
+    n, d = q.shape[1], q.shape[3]
+    cos, sin = hba_amd.rope_tables(n, d, 10000.0, dev)
+    scale = 1.0 / math.sqrt(d)
+    t = [x.to(dev) for x in (q, kx, v, gq, gk, idx, cnt, dout)]
+    kc, kr, vt = ops.prep_keys(t[1], t[2], t[4], 1e-6, cos, sin)
+    out = ops.attn_fwd(t[0], t[3], t[4], 1e-6, kc, kr, vt, cos, sin, t[5], t[6], S, W, scale)
+    got = ops.attn_bwd(t[0], t[1], t[2], kc, kr, t[3], t[4], 1e-6, cos, sin, t[5], t[6], out, t[7], S, W, scale)
+    return [x.cpu() for x in got], scale, cos.cpu().double(), sin.cpu().double()
+
+
+#           n    Hq Hkv  d   S   W   k
+BWD_SHAPES = [s for s in SHAPES if s[4] <= 64 and s[6] <= 64 and s[1] // s[2] <= 16] + [
+    (832, 3, 1, 64, 17, 300, 4),       # 5 queries per tile, two sink waves, ranges of 256 rows, the last one ragged
+    (4608, 2, 2, 64, 4, 70, 3),        # one head per KV head, ranges of 512 rows
+]
+
+
+@pytest.mark.parametrize("shape", BWD_SHAPES)
+def test_backward_against_64_bits(shape):
+    n, Hq, Hkv, d, S, W, k = shape
+    q, kx, v, gq, gk, idx, cnt = _inputs(*shape)
+    if n > 1024:
+        q, kx, v, idx, cnt = q[:1], kx[:1], v[:1], idx[:1], cnt[:1]
+    idx = _unique(idx, n)
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(5))
+    got, scale, cos, sin = _run_bwd(q, kx, v, gq, gk, idx, cnt, dout, S, W)
+    ref = _grads(q, kx, v, gq, gk, idx, cnt, dout, S, W, scale, cos, sin)
+    # p carries the logits' error of 1.7e-5 at most (see above) and dS = p (dP
+    # - D) cancels to about 1 / sqrt(keys) of its terms; a row with few keys
+    # keeps the sums' 2^-24 sqrt(terms).  In practice a tenth of this
+    for name, a, r in zip(("dq", "dk", "dv", "dgq", "dgk"), got, ref):
+        # rows that attend a single key have dS = 0 but for the rounding of dP
+        # - D, 2^-24 sqrt(d) |dO| |v| <= 1e-5 per element; the gains sum n rows
+        floor = 1e-5 * math.sqrt(r.numel()) * (math.sqrt(n * Hq / Hkv) if r.dim() == 1 else 1.0)
+        assert (a.double() - r).norm() <= 1e-5 * r.norm() + floor, name
+
+
+def test_backward_rows_outside_the_union_are_not_read_into_it():
+    """A NaN cotangent row reaches the keys it attends and a NaN key the
+    queries that attend it, and nothing else of their tiles."""
+    n, Hq, Hkv, d, S, W, k = shape = (320, 7, 1, 64, 4, 64, 2)
+    q, kx, v, gq, gk, idx, cnt = _inputs(*shape)
+    idx[:], cnt[:] = 0, 0
+    idx[:, :, 201, 0], cnt[:, :, 201] = 1, 1        # query 201 alone picks block 1
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(5))
+    bad = dout.clone()
+    bad[:, 201] = math.nan
+    got, scale, cos, sin = _run_bwd(q, kx, v, gq, gk, idx, cnt, bad, S, W)
+    ref = _grads(q, kx, v, gq, gk, idx, cnt, dout.index_fill(1, torch.tensor([201]), 0.0), S, W, scale, cos, sin)
+    j = torch.arange(n)
+    hit = (j < S) | ((j > 201 - W) & (j <= 201)) | ((j >= 64) & (j < 128))
+    for a, r, sel in ((got[0], ref[0], j == 201), (got[1], ref[1], hit), (got[2], ref[2], hit)):
+        assert a[:, sel].isnan().all()
+        assert (a[:, ~sel].double() - r[:, ~sel]).norm() <= 1e-5 * r.norm()
+    kb = kx.clone()
+    kb[:, 70] = math.nan                            # key 70: block 1, and the window of 70 .. 133
+    got = _run_bwd(q, kb, v, gq, gk, idx, cnt, dout, S, W)[0]
+    sel = ((j >= 70) & (j < 70 + W)) | (j == 201)
+    assert got[0][:, sel].isnan().all() and got[0][:, ~sel].isfinite().all()
