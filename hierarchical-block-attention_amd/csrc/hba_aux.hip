@@ -20,14 +20,14 @@
 //   aux_scores  grouped queries qg (fp32) and bsc with the tied-slot masks
 //   aux_teacher per (query, head, candidate block) the block LSE of the
 //               content logits, on MFMA (16 keys x 16 (query, head) columns;
-//               bf16: 16 waves share each staged key block)
+//               bf16: a workgroup shares each staged key block)
 //   aux_rows    per (query, KV head): p*, the row's KL term, d aux / d bsc
 //   aux_sum     aux = -(sum of row terms) / N, one workgroup, fixed order
 //   aux_dsum    d aux / d S0 = sum over queries of d bsc * tie share * qg
 //               (query segments, partials summed in order by aux_gsum)
 //   aux_sbwd    per block: the summariser's backward into per-block partial
 //               d probes / d proj
-//   aux_gsum    partials summed over blocks in a fixed order
+//   aux_bsum    partials summed over blocks in a fixed order
 // Every reduction runs in a fixed order: the results are deterministic.
 #include "hba_common.h"
 #include "hba_abi.h"
@@ -280,6 +280,18 @@ __global__ __launch_bounds__(256, 2) void aux_scores_mfma_kernel(const bf16_t *_
 }
 
 // ------------------------------------------------------------- teacher -----
+// Workgroup -> (query tile, KV head, batch) of both teachers: the last tiles
+// first, over all heads, since a tile's work grows with its candidate count
+// (in ascending order and head by head the compute units that began with the
+// longest tiles of one head also took the longest of the next: 2.14 ms for a
+// 32768-token call of 14 / 2 heads, head dim 64, against 1.74 in this order).
+__device__ __forceinline__ void teacher_tile(int64_t ntile, int64_t Hkv, int64_t &tile, int64_t &g, int64_t &b) {
+    const int64_t BH = gridDim.x / ntile, bg = blockIdx.x % BH;
+    tile = ntile - 1 - blockIdx.x / BH;
+    g = bg % Hkv;
+    b = bg / Hkv;
+}
+
 // Each wave owns 16 columns: QPW = 16/G queries x the G heads of KV head g
 // (column c -> query i0w + c/G, head g*G + c%G; columns past QPW*G idle).
 // For every candidate block of its last query it forms S^T = K_blk . Q^T as
@@ -297,10 +309,11 @@ __global__ __launch_bounds__(256) void aux_teacher_kernel(const typename St<DT>:
                                                           float *__restrict__ L) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int l16 = lane & 15, lg = lane >> 4;
-    const int64_t g = blockIdx.y, b = blockIdx.z;
     const int G = (int)(Hq / Hkv), QPW = 16 / G;
+    int64_t tile, g, b;
+    teacher_tile((n + 4 * QPW - 1) / (4 * QPW), Hkv, tile, g, b);
     const int64_t nb = n / BK;
-    const int64_t i0w = ((int64_t)blockIdx.x * 4 + w) * QPW;
+    const int64_t i0w = (tile * 4 + w) * QPW;
     if (i0w >= n) return;
     const int cq = l16 / G, ch = l16 % G;
     const int64_t iq = i0w + cq;
@@ -383,8 +396,8 @@ __global__ __launch_bounds__(256) void aux_teacher_kernel(const typename St<DT>:
     }
 }
 
-// bf16 teacher with the key blocks shared: a workgroup of 16 waves covers
-// 16 * CT * QPW consecutive queries (each wave CT column tiles of 16 columns,
+// bf16 teacher with the key blocks shared: a workgroup of TNW waves covers
+// TNW * CT * QPW consecutive queries (each wave CT column tiles of 16 columns,
 // QPW = 16/G queries x G heads each, so every A fragment read from LDS feeds
 // CT MFMAs) and streams the candidate blocks of its last query once through
 // a two-slot LDS buffer (rows padded to D + 8 bf16, so the 16 rows of an
@@ -393,23 +406,32 @@ __global__ __launch_bounds__(256) void aux_teacher_kernel(const typename St<DT>:
 // blocks past its own last query's candidates but meets every barrier.
 // Logits go through exp2 with scale * log2(e) folded into one multiply.
 constexpr int TCT = 2;   // column tiles per teacher wave
+// Waves per teacher workgroup.  The kernel is bound by its exponentials, so
+// what costs is waves that wait at the block's barrier: two workgroups of 8
+// waves on a compute unit cover each other's barriers, one of 16 (88 VGPRs do
+// not fit two) does not, and 4 waves share a staged block too little.  At
+// 32768 tokens, 14 / 2 heads, head dim 64: 1.55 ms with 8, 1.74 with 16, 2.47
+// with 4.
+constexpr int TNW = 8;
 
 template <int D>
-__global__ __launch_bounds__(1024) void aux_teacher_bf16_kernel(const bf16_t *__restrict__ qc,
+__global__ __launch_bounds__(64 * TNW) void aux_teacher_bf16_kernel(const bf16_t *__restrict__ qc,
                                                                 const bf16_t *__restrict__ kc, int64_t n,
                                                                 int64_t Hq, int64_t Hkv, int64_t W, float scale_u,
                                                                 const float *__restrict__ qgain,
                                                                 const float *__restrict__ kgain,
                                                                 float *__restrict__ L) {
-    constexpr int NW = 16, NKS = D / 32, ROW = D + 8, CH = BK * D / 8;   // CH 16-byte chunks per block
-    static_assert(CH <= NW * 64, "one chunk per thread");
+    constexpr int NW = TNW, NKS = D / 32, ROW = D + 8;
+    constexpr int CPT = BK * D / 8 / (64 * NW);   // 16-byte chunks of a block per thread
+    static_assert(CPT * 64 * NW == BK * D / 8, "whole chunks per thread");
     __shared__ __align__(16) bf16_t kb[2][BK * ROW];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int l16 = lane & 15, lg = lane >> 4;
-    const int64_t g = blockIdx.y, b = blockIdx.z;
     const int G = (int)(Hq / Hkv), QPW = 16 / G;
+    int64_t tile, g, b;
+    teacher_tile((n + NW * TCT * QPW - 1) / (NW * TCT * QPW), Hkv, tile, g, b);
     const int64_t nb = n / BK;
-    const int64_t i0 = (int64_t)blockIdx.x * NW * TCT * QPW;
+    const int64_t i0 = tile * NW * TCT * QPW;
     const int64_t ilast = (i0 + NW * TCT * QPW - 1 < n) ? i0 + NW * TCT * QPW - 1 : n - 1;
     const int64_t bmax = cand_bmax(ilast, BK, W);          // uniform over the workgroup
     if (bmax < 1) return;
@@ -445,14 +467,24 @@ __global__ __launch_bounds__(1024) void aux_teacher_bf16_kernel(const bf16_t *__
         }
     }
     const bf16_t *kg = kc + (b * Hkv + g) * n * D;
-    const bool ld = tid < CH;
     const int r = tid / (D / 8), cc = tid % (D / 8);
-    uint4 reg = ld ? *reinterpret_cast<const uint4 *>(kg + (BK + r) * D + 8 * cc) : make_uint4(0, 0, 0, 0);
+    constexpr int RPP = 64 * NW / (D / 8);   // rows between a thread's chunks
+    uint4 reg[CPT];
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) reg[u] = *reinterpret_cast<const uint4 *>(kg + (BK + r + u * RPP) * D + 8 * cc);
+    float keep[TCT];   // the LSE of the block c with c % 4 = lg, stored when c % 4 = 3: 16 bytes per column
+#pragma unroll
+    for (int t = 0; t < TCT; ++t) keep[t] = 0.0f;
     for (int64_t c = 1; c <= bmax; ++c) {
         bf16_t *slot = kb[c & 1];
-        if (ld) *reinterpret_cast<uint4 *>(slot + r * ROW + 8 * cc) = reg;
+#pragma unroll
+        for (int u = 0; u < CPT; ++u) *reinterpret_cast<uint4 *>(slot + (r + u * RPP) * ROW + 8 * cc) = reg[u];
         __syncthreads();   // this block staged; every wave is past block c - 2, which used this slot
-        if (ld && c + 1 <= bmax) reg = *reinterpret_cast<const uint4 *>(kg + ((c + 1) * BK + r) * D + 8 * cc);
+        if (c + 1 <= bmax) {
+#pragma unroll
+            for (int u = 0; u < CPT; ++u)
+                reg[u] = *reinterpret_cast<const uint4 *>(kg + ((c + 1) * BK + r + u * RPP) * D + 8 * cc);
+        }
         if (c > wmax) continue;
         f32x4 acc[TCT][4];
 #pragma unroll
@@ -487,16 +519,95 @@ __global__ __launch_bounds__(1024) void aux_teacher_bf16_kernel(const bf16_t *__
                 for (int e = 0; e < 4; ++e) se += __builtin_amdgcn_exp2f(fmaf(acc[t][mt][e], s2, -off));
             se += __shfl_xor(se, 16, 64);
             se += __shfl_xor(se, 32, 64);
-            if (lg == 0 && col_ok[t] && c <= col_bmax[t]) Lrow[t][c] = (off + __log2f(se)) * 0.6931471805599453f;
+            if ((c & 3) == lg) keep[t] = (off + __log2f(se)) * 0.6931471805599453f;
+            const int64_t cl = (c & ~(int64_t)3) + lg;
+            if (((c & 3) == 3 || c == wmax) && cl >= 1 && cl <= c && cl <= col_bmax[t]) Lrow[t][cl] = keep[t];
         }
     }
 }
 
 // ---------------------------------------------------------------- rows -----
 // One wave per (b, g, i) with a candidate block: p* from the block LSEs, the
-// row's KL term (rowt), and d aux / d bsc written over bsc.  Head h's max and
-// sum of exponentials over the candidate blocks are kept by lane h.
-__global__ __launch_bounds__(256) void aux_rows_kernel(float *__restrict__ L, int64_t B, int64_t n,
+// row's KL term (rowt), and d aux / d bsc written over bsc.  Bound by its one
+// read of L.  Up to 64 R candidate blocks (R is the smallest of 4, 8, 16 that
+// holds them) a lane keeps its blocks' values in registers; more take three
+// passes over L, with p(c) in place of head 0's values.  At 32768 tokens, 14 /
+// 2 heads: 440 us with the passes over L, 167 us with the registers.
+template <int R>
+__global__ __launch_bounds__(256) void aux_rows_kernel(const float *__restrict__ L, int64_t B, int64_t n, int64_t Hkv,
+                                                       int G, int64_t W, float invN, float *__restrict__ bsc,
+                                                       float *__restrict__ rowt) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t r = (int64_t)blockIdx.x * 4 + w;
+    if (r >= B * Hkv * n) return;
+    const int64_t i = r % n;
+    const int64_t nb = n / BK;
+    const int nbm = (int)cand_bmax(i, BK, W);
+    if (nbm < 1) {
+        if (lane == 0) rowt[r] = 0.0f;
+        return;
+    }
+    const float *Lr = L + r * G * nb;
+    float *br = bsc + r * nb;
+    float p[R], v[R];
+#pragma unroll
+    for (int t = 0; t < R; ++t) p[t] = 0.0f;
+    for (int h = 0; h < G; ++h) {   // softmax over the blocks, added to the group's sum
+        float mx = -INFINITY, z = 0.0f;
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const int c = 1 + lane + 64 * t;
+            v[t] = (c <= nbm) ? Lr[h * nb + c] : -INFINITY;
+            mx = fmaxf(mx, v[t]);
+        }
+        mx = wave_max(mx);
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            v[t] = (1 + lane + 64 * t <= nbm) ? expf(v[t] - mx) : 0.0f;
+            z += v[t];
+        }
+        z = wave_sum(z);
+        const float rz = 1.0f / z;
+#pragma unroll
+        for (int t = 0; t < R; ++t) p[t] = fmaf(v[t], rz, p[t]);
+    }
+    float p0 = 0.0f, top = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+        const int c = 1 + lane + 64 * t;
+        p[t] /= (float)G;
+        p0 += p[t];
+        v[t] = (c <= nbm) ? br[c] : -INFINITY;
+        top = fmaxf(top, v[t]);
+    }
+    p0 = fmaxf(wave_sum(p0), 1e-9f);
+    top = wave_max(top);
+    float zb = 0.0f;
+#pragma unroll
+    for (int t = 0; t < R; ++t) zb += (1 + lane + 64 * t <= nbm) ? expf(v[t] - top) : 0.0f;
+    const float lse = top + logf(wave_sum(zb));
+    float term = 0.0f, P = 0.0f;
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+        p[t] /= p0;
+        if (p[t] > 0.0f) {
+            term += p[t] * (v[t] - lse);
+            P += p[t];
+        }
+    }
+    term = wave_sum(term);
+    P = wave_sum(P);
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+        const int c = 1 + lane + 64 * t;
+        if (c <= nbm) br[c] = (expf(v[t] - lse) * P - (p[t] > 0.0f ? p[t] : 0.0f)) * invN;
+    }
+    if (lane == 0) rowt[r] = term;
+}
+
+// The passes over L.  Head h's max and sum of exponentials over the candidate
+// blocks are kept by lane h.
+__global__ __launch_bounds__(256) void aux_rows_long_kernel(float *__restrict__ L, int64_t B, int64_t n,
                                                        int64_t Hkv, int G, int64_t W, float invN,
                                                        float *__restrict__ bsc, float *__restrict__ rowt) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -571,15 +682,22 @@ __global__ __launch_bounds__(256) void aux_rows_kernel(float *__restrict__ L, in
 }
 
 // aux = -(sum of the row terms) / N: one workgroup, double accumulation in a
-// fixed order.
-__global__ __launch_bounds__(256) void aux_sum_kernel(const float *__restrict__ rowt, int64_t rows, float invN,
-                                                      float *__restrict__ aux) {
-    __shared__ double part[256];
+// fixed order; eight loads in flight per thread (65536 rows: 88 us with one
+// load at a time and 256 threads, 23 us so).
+__global__ __launch_bounds__(1024) void aux_sum_kernel(const float *__restrict__ rowt, int64_t rows, float invN,
+                                                       float *__restrict__ aux) {
+    __shared__ double part[1024];
     double s = 0.0;
-    for (int64_t r = threadIdx.x; r < rows; r += 256) s += (double)rowt[r];
+    for (int64_t r0 = threadIdx.x; r0 < rows; r0 += 8 * 1024) {
+        float x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = (r0 + 1024 * u < rows) ? rowt[r0 + 1024 * u] : 0.0f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += (double)x[u];
+    }
     part[threadIdx.x] = s;
     __syncthreads();
-    for (int o = 128; o >= 1; o >>= 1) {
+    for (int o = 512; o >= 1; o >>= 1) {
         if ((int)threadIdx.x < o) part[threadIdx.x] += part[threadIdx.x + o];
         __syncthreads();
     }
@@ -860,8 +978,8 @@ __global__ __launch_bounds__(256) void aux_sbwd_kernel(const typename St<DT>::T 
     }
 }
 
-// Sum of per-block partials (count of them, each `len` floats apart) in block
-// order.
+// Sum of the query segments' partials (count of them, each `len` floats
+// apart) in order.
 __global__ __launch_bounds__(256) void aux_gsum_kernel(const float *__restrict__ part, int64_t count,
                                                        int64_t len, float *__restrict__ out) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -869,6 +987,38 @@ __global__ __launch_bounds__(256) void aux_gsum_kernel(const float *__restrict__
     float s = 0.0f;
     for (int64_t p = 0; p < count; ++p) s += part[p * len + e];
     out[e] = s;
+}
+
+// d proj and d probes from their per-block partials: a workgroup takes 64
+// elements of one of them, wave w the w-th sixteenth of the blocks, eight
+// loads in flight; the waves' sums are added in order.  One thread per element
+// with its chain of `count` loads took 110 us for each of the two at 512
+// blocks; the one launch takes 5 us.
+__global__ __launch_bounds__(1024) void aux_bsum_kernel(const float *__restrict__ pproj, const float *__restrict__ pprb,
+                                                        int64_t count, int64_t lp, int64_t lb,
+                                                        float *__restrict__ dproj, float *__restrict__ dprobes) {
+    __shared__ float part[16][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const bool prb = (int64_t)blockIdx.x * 64 >= lp;
+    const int64_t len = prb ? lb : lp, e = (int64_t)blockIdx.x * 64 - (prb ? lp : 0) + lane;
+    const float *src = (prb ? pprb : pproj) + e;
+    const int64_t per = (count + 15) / 16, c0 = w * per, c1 = (c0 + per < count) ? c0 + per : count;
+    float s = 0.0f;
+    for (int64_t c = c0; c < c1; c += 8) {
+        float x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = (c + u < c1) ? src[(c + u) * len] : 0.0f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += x[u];
+    }
+    part[w][lane] = s;
+    __syncthreads();
+    if (w == 0) {
+        float t = part[0][lane];
+#pragma unroll
+        for (int u = 1; u < 16; ++u) t += part[u][lane];
+        (prb ? dprobes : dproj)[e] = t;
+    }
 }
 
 __global__ void aux_zero_kernel(float *__restrict__ p, int64_t len) {
@@ -965,21 +1115,28 @@ extern "C" int hba_aux_kl(int dtype, const void *q, const int64_t q_strides[3], 
         const int64_t qpw = 16 / G;                                                                      \
         if (DT == 1)                                                                                     \
             hipLaunchKernelGGL((aux::aux_teacher_bf16_kernel<D>),                                        \
-                               dim3((unsigned)((n + 16 * aux::TCT * qpw - 1) / (16 * aux::TCT * qpw)),    \
-                                    (unsigned)Hkv,                                                       \
-                               (unsigned)B), dim3(1024), 0, s, (const bf16_t *)qc, (const bf16_t *)kc, n,  \
+                               dim3((unsigned)((n + aux::TNW * aux::TCT * qpw - 1) / (aux::TNW * aux::TCT * qpw) * Hkv * B)), \
+                               dim3(64 * aux::TNW), 0, s, (const bf16_t *)qc, (const bf16_t *)kc, n,  \
                                Hq, Hkv, W, scale_u, q_gain, k_gain, Lb);                                 \
         else                                                                                             \
             hipLaunchKernelGGL((aux::aux_teacher_kernel<DT, D>),                                         \
-                               dim3((unsigned)((n + 4 * qpw - 1) / (4 * qpw)), (unsigned)Hkv,             \
-                               (unsigned)B), dim3(256), 0, s, (const T *)qc, (const T *)kc, n, Hq, Hkv, W, \
+                               dim3((unsigned)((n + 4 * qpw - 1) / (4 * qpw) * Hkv * B)), dim3(256), 0, s, \
+                               (const T *)qc, (const T *)kc, n, Hq, Hkv, W, \
                                scale_u, Lb);                                                             \
     } while (0)
     HBA_DISPATCH_DT_D(dtype, d, HBA_AUX_FWD);
 #undef HBA_AUX_FWD
-    hipLaunchKernelGGL(aux::aux_rows_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, Lb, B, n, Hkv,
-                       (int)G, W, invN, bsc, rowt);
-    hipLaunchKernelGGL(aux::aux_sum_kernel, dim3(1), dim3(256), 0, s, rowt, rows, invN, aux);
+    const int64_t ncand = cand_bmax(n - 1, aux::BK, W);
+    if (ncand <= 64 * 16) {
+        const auto kern = ncand <= 64 * 4 ? aux::aux_rows_kernel<4>
+                                          : ncand <= 64 * 8 ? aux::aux_rows_kernel<8> : aux::aux_rows_kernel<16>;
+        hipLaunchKernelGGL(kern, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, Lb, B, n, Hkv, (int)G, W, invN, bsc,
+                           rowt);
+    } else {
+        hipLaunchKernelGGL(aux::aux_rows_long_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, Lb, B, n, Hkv,
+                           (int)G, W, invN, bsc, rowt);
+    }
+    hipLaunchKernelGGL(aux::aux_sum_kernel, dim3(1), dim3(1024), 0, s, rowt, rows, invN, aux);
     if (dprobes) {
 #define HBA_AUX_BWD(DT, D)                                                                               \
     do {                                                                                                 \
@@ -1004,10 +1161,9 @@ extern "C" int hba_aux_kl(int dtype, const void *q, const int64_t q_strides[3], 
         HBA_DISPATCH_DT_D(dtype, d, HBA_AUX_BWD);
 #undef HBA_AUX_BWD
         const int64_t lp = Hkv * d * d, lb = Hkv * m * d;
-        hipLaunchKernelGGL(aux::aux_gsum_kernel, dim3((unsigned)((lp + 255) / 256)), dim3(256), 0, s, pproj, B * nb,
-                           lp, dproj);
-        hipLaunchKernelGGL(aux::aux_gsum_kernel, dim3((unsigned)((lb + 255) / 256)), dim3(256), 0, s, pprb, B * nb,
-                           lb, dprobes);
+        // both are whole numbers of 64 elements (d is 64 or 128)
+        hipLaunchKernelGGL(aux::aux_bsum_kernel, dim3((unsigned)((lp + lb) / 64)), dim3(1024), 0, s, pproj, pprb,
+                           B * nb, lp, lb, dproj, dprobes);
     }
     HBA_LAUNCH_CHECK();
     return HBA_OK;
