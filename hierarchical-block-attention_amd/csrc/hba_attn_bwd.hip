@@ -95,7 +95,7 @@ __device__ __forceinline__ bf16x8 ld_b8(const bf16_t *p) {
 __device__ __forceinline__ bf16x8 pack_b8(const float (&x)[8]) {
     u32x4b u;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) u[e] = (uint32_t)f2bf(x[2 * e]) | ((uint32_t)f2bf(x[2 * e + 1]) << 16);
+    for (int e = 0; e < 4; ++e) u[e] = pk_bf16(x[2 * e], x[2 * e + 1]);
     return __builtin_bit_cast(bf16x8, u);
 }
 __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
@@ -507,15 +507,15 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dq_mfma_kernel(
 
 // ------------------------------------------------ bwd_dkv on MFMA (bf16) ----
 // dK and dV of one 64-key block from the (query row, head) pairs that attend
-// it, 64 pairs per tile staged in LDS twice (row-major and transposed), taken
+// it, 64 pairs per tile staged in LDS, taken
 // as two halves of 32 (the contraction of one product); wave w
 // owns keys kb + 16 w .. kb + 16 w + 15:
 //   S   = X . K^T    (A: staged query rows X, pairs in the slot order pslot;
 //                     B: the wave's key rows, held in registers)
 //   dP  = dO . V^T   (A: staged dO rows; B: the wave's V rows)
 //   dV += P^T . dO   (A: P^T straight from the accumulators, which the slot
-//                     order puts in the A-operand layout; B: dO^T from the
-//                     transposed copy)
+//                     order puts in the A-operand layout; B: dO^T by
+//                     transposing LDS reads, ld_tr8)
 //   dK += dS^T . X   (A: dS^T the same way; B: X^T)
 // Lane (l16, lg) holds S and dP of key l16 and pairs 8 lg + 4 mt + e, and of
 // dV / dK the element d = 16 dt + l16 of keys 16 w + 4 lg + e.
@@ -525,6 +525,13 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dq_mfma_kernel(
 // (fp32 atomics) into dkv_acc [B, Hkv, n, 3, d] (NoPE dk, rotated dk, dv),
 // which bwd_dkv_fin turns into dk and dv.  The split over row ranges keeps a
 // block that nearly every query selects from becoming the tail.
+// Bound by VALU issue and LDS reads together (45 % and 60 % of its time).  At
+// 32768 tokens, 14 / 2 heads, head dim 64: 1.52 ms with a second, transposed
+// copy of each tile (2-byte LDS stores), 1.42 with the transposing reads, 1.09
+// with pair indexes and masks in 32 bits, no masks where a half's rows attend
+// all of the wave's keys, one fma per exponent and packed bf16 conversions.
+// Transposing reads take twice the cycles of plain ones, in padded rows as in
+// rows of permuted chunks (1.12 ms).
 // With sink_rows > 0 the launch takes the sink keys instead: one workgroup
 // per (b, g, range of sink_rows rows) against block 0, every row of the range
 // attending the keys j < S with j <= i (NoPE); waves whose 16 keys hold no
@@ -533,16 +540,26 @@ constexpr int SINK_ROWS = 256;   // query rows per workgroup of the sink launch
 constexpr int DKV_RL = 1024;   // routed rows run as one series of tiles at most
 constexpr int DKV_TP = 64;   // pairs per tile: two halves of 32, the pair count of one product
 
+// Elements 8 lg .. + 7 of a column of a row-major LDS tile: ds_read_b64_tr_b16
+// gives lane r of 16 the elements r % 4 of the four 8-byte pieces that lanes
+// r / 4 + 4 j (j = 0 .. 3) address, so lane r addresses columns 4 (r % 4) .. + 3
+// of row r / 4 (p0: of rows 0 .. 3, p1: of rows 4 .. 7) and receives column r.
+__device__ __forceinline__ bf16x8 ld_tr8(const bf16_t *p0, const bf16_t *p1) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    typedef __attribute__((address_space(3))) s16x4 *lds4;
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)p0);
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)p1);
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
 __device__ __forceinline__ int pslot(int mt, int r) { return 8 * (r >> 2) + 4 * mt + (r & 3); }
 
 template <int D>
 struct DkvTile {
-    static constexpr int XP = D + 8;        // padded row of the row-major copies
-    static constexpr int TP = DKV_TP + 8;   // padded row of the transposed copies
+    static constexpr int XP = D + 8;        // padded row
     alignas(16) bf16_t xs[DKV_TP * XP];
     alignas(16) bf16_t os[DKV_TP * XP];
-    alignas(16) bf16_t xt[D * TP];
-    alignas(16) bf16_t ot[D * TP];
     alignas(16) float lse[DKV_TP];
     alignas(16) float dd[DKV_TP];
     alignas(16) int row[DKV_TP];
@@ -564,7 +581,7 @@ __global__ __launch_bounds__(DKV_NT, D == 64 ? 4 : 2) void bwd_dkv_mfma_kernel(
     constexpr int NKS = D / 32, NDT = D / 16, NCH = D / 8, CPT = DKV_TP * NCH / DKV_NT;
     static_assert(CPT * DKV_NT == DKV_TP * NCH, "a tile's 16-byte chunks split evenly over the threads");
     using Tl = DkvTile<D>;
-    constexpr int XP = Tl::XP, TP = Tl::TP;
+    constexpr int XP = Tl::XP;
     __shared__ Tl tl[2];
     __shared__ int rows[DKV_RL];
     __shared__ int wcount[DKV_NT / 64];
@@ -581,6 +598,9 @@ __global__ __launch_bounds__(DKV_NT, D == 64 ? 4 : 2) void bwd_dkv_mfma_kernel(
     const int64_t rows_per = sinks ? (int64_t)sink_rows : (int64_t)DKV_ROWS;
     const int64_t r0 = (int64_t)split * rows_per, r1 = min(n, r0 + rows_per);
     const int64_t jl = kb + 16 * kg + l16;   // the key of this lane's S / dP column
+    const int Wc = (int)min(W, n);           // past n a longer window changes nothing
+    const float sl2 = scale * 1.4426950408889634f;
+    const uint32_t gmagic = 0xffffffffu / (uint32_t)G + 1u;   // G > 1: u / G = umulhi(u, gmagic) for u < 2^28
 
     // the key operand of the current rows (kr rows for the window, kc rows
     // for the sinks and routed rows) and the value rows
@@ -625,32 +645,33 @@ __global__ __launch_bounds__(DKV_NT, D == 64 ? 4 : 2) void bwd_dkv_mfma_kernel(
 
     // pairs gp = 0 .. total-1: query row row_of(gp / G), head g G + gp % G;
     // mode 0: window rows (rotated), 1: routed rows, 2: sink rows (NoPE)
-    auto run = [&](int64_t total, auto row_of, int mode) {
+    auto run = [&](int total, auto row_of, int mode) {
         const bool rope = mode == 0;
         const bf16_t *qx = rope ? qr_ws : qc_ws;
-        const int64_t ntl = (total + DKV_TP - 1) / DKV_TP;
+        const int ntl = (total + DKV_TP - 1) / DKV_TP;
         u32x4b xr[CPT], orr[CPT];
         float plse[CPT], pdd[CPT];
         int prow[CPT];
-        auto load = [&](int64_t t) {
+        auto load = [&](int t) {
 #pragma unroll
             for (int r = 0; r < CPT; ++r) {
                 const int q = tid + DKV_NT * r, p = q / NCH, c = q % NCH;
-                const int64_t gp = t * DKV_TP + p;
+                const int gp = t * DKV_TP + p;
                 plse[r] = INFINITY;
                 pdd[r] = 0.0f;
                 prow[r] = -1;
                 if (gp < total) {
-                    const int64_t i = row_of(gp / G);
-                    const int h = g * G + (int)(gp % G);
+                    const int rr = (G == 1) ? gp : (int)__umulhi((uint32_t)gp, gmagic);
+                    const int i = row_of(rr);
+                    const int h = g * G + gp - rr * G;
                     const int64_t ro = (((int64_t)b * n + i) * Hq + h) * D + 8 * c;
                     xr[r] = *reinterpret_cast<const u32x4b *>(qx + ro);
                     orr[r] = *reinterpret_cast<const u32x4b *>(dout + ro);
                     if (c == 0) {
                         const int64_t so = ((int64_t)b * Hq + h) * n + i;
-                        plse[r] = lse_ws[so];
+                        plse[r] = lse_ws[so] * 1.4426950408889634f;
                         pdd[r] = dd_ws[so];
-                        prow[r] = (int)i;
+                        prow[r] = i;
                     }
                 } else {
                     xr[r] = orr[r] = u32x4b{0u, 0u, 0u, 0u};
@@ -663,13 +684,6 @@ __global__ __launch_bounds__(DKV_NT, D == 64 ? 4 : 2) void bwd_dkv_mfma_kernel(
                 const int q = tid + DKV_NT * r, p = q / NCH, c = q % NCH;
                 *reinterpret_cast<u32x4b *>(&T.xs[p * XP + 8 * c]) = xr[r];
                 *reinterpret_cast<u32x4b *>(&T.os[p * XP + 8 * c]) = orr[r];
-                // transposed rows d = 8 c + e, this pair in 8-pair group (p >> 3) ^ (c & 7)
-                const int tc = ((((p >> 3) ^ c) & 7) << 3) | (p & 7);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    T.xt[(8 * c + e) * TP + tc] = (bf16_t)(xr[r][e >> 1] >> (16 * (e & 1)));
-                    T.ot[(8 * c + e) * TP + tc] = (bf16_t)(orr[r][e >> 1] >> (16 * (e & 1)));
-                }
                 if (c == 0) {
                     T.lse[p] = plse[r];
                     T.dd[p] = pdd[r];
@@ -695,20 +709,36 @@ __global__ __launch_bounds__(DKV_NT, D == 64 ? 4 : 2) void bwd_dkv_mfma_kernel(
                 }
             }
             float pk[8], dk[8];
+            // window rows ascend: the half's first and last say whether every
+            // pair attends every key of the wave (jw .. jw + 15)
+            const int jw = (int)kb + 16 * kg, jl = jw + l16;
+            const int i1 = T.row[32 * hp + 31];
+            const bool all = (mode == 1) ? i1 >= 0
+                             : (mode == 0) ? (jw >= S && T.row[32 * hp] >= jw + 15 && i1 >= 0 && i1 - jw < Wc)
+                                           : false;
 #pragma unroll
             for (int mt = 0; mt < 2; ++mt) {
                 const int pp = 32 * hp + 8 * lg + 4 * mt;
                 const f32x4 ls = *reinterpret_cast<const f32x4 *>(&T.lse[pp]);
                 const f32x4 ds = *reinterpret_cast<const f32x4 *>(&T.dd[pp]);
-                const int4 rw = *reinterpret_cast<const int4 *>(&T.row[pp]);
-                const int ri[4] = {rw.x, rw.y, rw.z, rw.w};
+                float arg[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) arg[e] = fmaf(Sa[mt][e], sl2, -ls[e]);
+                if (!__builtin_amdgcn_readfirstlane((int)all)) {
+                    const int4 rw = *reinterpret_cast<const int4 *>(&T.row[pp]);
+                    const int ri[4] = {rw.x, rw.y, rw.z, rw.w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int i = ri[e];
+                        const bool valid = (mode == 0) ? (jl >= S && i >= jl && i - jl < Wc)
+                                         : (mode == 1) ? (i >= 0)
+                                                       : (jl < S && i >= jl);
+                        arg[e] = valid ? arg[e] : -INFINITY;
+                    }
+                }
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int64_t i = ri[e];
-                    const bool valid = (mode == 0) ? (jl >= S && i >= jl && i <= jl + W - 1)
-                                     : (mode == 1) ? (i >= 0)
-                                                   : (jl < S && i >= jl);
-                    const float p = valid ? __expf(Sa[mt][e] * scale - ls[e]) : 0.0f;
+                    const float p = __builtin_amdgcn_exp2f(arg[e]);
                     pk[4 * mt + e] = p;
                     dk[4 * mt + e] = p * (Pa[mt][e] - ds[e]) * scale;
                 }
@@ -716,10 +746,10 @@ __global__ __launch_bounds__(DKV_NT, D == 64 ? 4 : 2) void bwd_dkv_mfma_kernel(
             const bf16x8 pa = pack_b8(pk), da = pack_b8(dk);
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) {
-                const int dr = 16 * dt + l16;                      // pairs 32 hp + 8 lg .. + 7 of row dr
-                const int to = dr * TP + ((((4 * hp + lg) ^ (dr >> 3)) & 7) << 3);
-                gv[dt] = mfma16(pa, ld_b8(&T.ot[to]), gv[dt]);
-                gk[dt] = mfma16(da, ld_b8(&T.xt[to]), gk[dt]);
+                // pairs 32 hp + 8 lg .. + 7 of element 16 dt + l16
+                const int to = (32 * hp + 8 * lg + (l16 >> 2)) * XP + 16 * dt + 4 * (l16 & 3);
+                gv[dt] = mfma16(pa, ld_tr8(&T.os[to], &T.os[to + 4 * XP]), gv[dt]);
+                gk[dt] = mfma16(da, ld_tr8(&T.xs[to], &T.xs[to + 4 * XP]), gk[dt]);
             }
           }
         };
@@ -727,7 +757,7 @@ __global__ __launch_bounds__(DKV_NT, D == 64 ? 4 : 2) void bwd_dkv_mfma_kernel(
         load(0);
         store(tl[0]);
         __syncthreads();
-        for (int64_t t = 0; t < ntl; ++t) {
+        for (int t = 0; t < ntl; ++t) {
             if (t + 1 < ntl) load(t + 1);
             compute(tl[t & 1]);
             if (t + 1 < ntl) store(tl[(t + 1) & 1]);
@@ -739,7 +769,7 @@ __global__ __launch_bounds__(DKV_NT, D == 64 ? 4 : 2) void bwd_dkv_mfma_kernel(
     if (sinks) {
         had_rt = true;
         load_k(kc);
-        run((r1 - r0) * G, [&](int64_t r) { return r0 + r; }, 2);
+        run((int)(r1 - r0) * G, [&](int r) { return (int)r0 + r; }, 2);
     }
     // window rows: key j >= S is in the window of queries j .. j + W - 1
     if (!sinks) {
@@ -748,7 +778,7 @@ __global__ __launch_bounds__(DKV_NT, D == 64 ? 4 : 2) void bwd_dkv_mfma_kernel(
         if (wb >= wa) {
             had_win = true;
             load_k(kr);
-            run((wb - wa + 1) * G, [&](int64_t r) { return wa + r; }, 0);
+            run((int)(wb - wa + 1) * G, [&](int r) { return (int)wa + r; }, 0);
             rope_t();
         }
     }
@@ -785,7 +815,7 @@ __global__ __launch_bounds__(DKV_NT, D == 64 ? 4 : 2) void bwd_dkv_mfma_kernel(
             __syncthreads();                                      // rows[] complete
             had_rt = true;
             const int tot = min(DKV_RL, total - run0);
-            run((int64_t)tot * G, [&](int64_t r) { return (int64_t)rows[r]; }, 1);
+            run(tot * G, [&](int r) { return rows[r]; }, 1);
         }
     }
 
