@@ -1194,26 +1194,30 @@ __global__ __launch_bounds__(RtCfg<D>::NTHR, RtCfg<D>::NTHR / 256) void attn_rou
 // (the gradient with respect to the QKNorm'd row; window keys give it in the
 // rotated frame).  Per 64-key block: S^T = K.Q^T and dP^T = V.dO^T (K and V
 // tiles, key rows in permk order, so that both accumulators come out in the
-// B-operand layout), then dq^T += K^T.dS^T (K^T tile).  A ring slot holds
-// the three tiles.  The window tiles (kr, krt; the RoPE operand) stream
+// B-operand layout), then dq^T += K^T.dS^T (K^T by transposing reads of the K
+// tile).  A ring slot holds the two tiles.  The window tiles (kr; the RoPE operand) stream
 // first; rope^T then maps the column's partial sum back to the unrotated
 // frame in registers (a row element and its rotation partner sit in the same
-// lane) and the sinks and routed blocks (kc, kct; the NoPE operand, read back
+// lane) and the sinks and routed blocks (kc; the NoPE operand, read back
 // from the rows this workgroup wrote at set-up) follow in the same softmax
 // state.  Softmax as the forward: the QKNorm bound as a fixed shift when it
 // holds, else a running max.  Outputs: dq (rope^T and the QKNorm backward
 // applied), the gain gradient (one atomic per head per workgroup), and for
 // the key-gradient kernels the QKNorm'd and rotated rows (bf16), the LSE
 // (natural log) and D.
+//
+// No VGPR may spill here: the compiler has placed the spill of a value that
+// lives past a divergent loop before the loop's exec restore, where it stores
+// nothing (the LSE rows of a build with 16 spilled VGPRs all went to head 0).
 template <int D, int WAVES>
 struct DqCfg {
     static constexpr int NKS = D / 32;
     static constexpr int NDT = D / 16;
     static constexpr int NTHR = WAVES * 64;
-    static constexpr int TILE = 64 * D;                   // bf16 elements of a K, V or K^T tile
-    static constexpr int SLOT = 3 * TILE;
+    static constexpr int TILE = 64 * D;                   // bf16 elements of a K or V tile
+    static constexpr int SLOT = 2 * TILE;
     static constexpr int KPARTS = TILE * 2 / 1024;        // 1 KB parts of a tile
-    static constexpr int NPARTS = 3 * KPARTS;
+    static constexpr int NPARTS = 2 * KPARTS;
     static constexpr int PPW = (NPARTS + WAVES - 1) / WAVES;   // DMA parts per wave per block, at most
 };
 
@@ -1236,9 +1240,8 @@ __device__ __forceinline__ bf16x8 scale8(bf16x8 x, float f) {
 // after the scores' exponentials, so that the K and V fragments are not live
 // together.
 template <int D, bool FIXED, int MODE>
-__device__ __forceinline__ void dq_update(const bf16_t *Ks, const bf16_t *Vk, const bf16_t *KT,
-                                          const bf16x8 (&qop)[D / 32], const bf16x8 (&dop)[D / 32], float Dh,
-                                          f32x4 (&acc)[D / 16], float &mrun, float &lsum, bool colok, int jlo,
+__device__ __forceinline__ void dq_update(const bf16_t *Ks, const bf16_t *Vk, const bf16x8 (&qop)[D / 32],
+                                          const bf16x8 (&dop)[D / 32], float Dh, f32x4 (&acc)[D / 16], float &mrun, float &lsum, bool colok, int jlo,
                                           int jhi, float sl2, float bl2, int l16, int lg) {
     constexpr int NKS = D / 32, NDT = D / 16;
     asm volatile("" ::: "memory");   // no fragment held over from the previous row tile
@@ -1309,21 +1312,22 @@ __device__ __forceinline__ void dq_update(const bf16_t *Ks, const bf16_t *Vk, co
             ds[mt >> 1][(mt & 1) * 4 + e] = p[mt][e] * (Pa[mt][e] - Dh);
         }
     const bf16x8 db0 = pack8(ds[0]), db1 = pack8(ds[1]);
-    const int swt = swzV(l16);   // swzV(16 dt + l16) for every dt
+    // K^T fragments: keys 8 lg .. + 7 (and 32 on) of element 16 dt + l16; the
+    // four rows this lane addresses (r0, + 4, + 32, + 36) share one swizzle
+    const int r0 = 8 * lg + (l16 >> 2), swr = swzK(r0);
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) {
-        const bf16_t *kp = KT + (16 * dt + l16) * 64;
-        acc[dt] = mma(ldb8(kp + 8 * (lg ^ swt)), db0, acc[dt]);
-        acc[dt] = mma(ldb8(kp + 8 * ((lg + 4) ^ swt)), db1, acc[dt]);
+        const bf16_t *kp = Ks + r0 * D + 8 * ((2 * dt + ((l16 >> 1) & 1)) ^ swr) + 4 * (l16 & 1);
+        acc[dt] = mma(ld_tr8(kp, kp + 4 * D), db0, acc[dt]);
+        acc[dt] = mma(ld_tr8(kp + 32 * D, kp + 36 * D), db1, acc[dt]);
     }
 }
 
 template <int D, int WAVES, int PTW, int NS, int PH, bool FIXED>
 __device__ __forceinline__ void dq_body(
     const bf16_t *__restrict__ q, const float *__restrict__ qgain, float eps, const bf16_t *__restrict__ kc,
-    const bf16_t *__restrict__ kr, const bf16_t *__restrict__ kct, const bf16_t *__restrict__ krt,
-    const bf16_t *__restrict__ v, const float *__restrict__ cosT, const float *__restrict__ sinT,
-    const int32_t *__restrict__ idx, const int32_t *__restrict__ cnt, const bf16_t *__restrict__ out,
+    const bf16_t *__restrict__ kr, const bf16_t *__restrict__ v, const float *__restrict__ cosT,
+    const float *__restrict__ sinT, const int32_t *__restrict__ idx, const int32_t *__restrict__ cnt, const bf16_t *__restrict__ out,
     const bf16_t *__restrict__ dout, int64_t n, int Hq, int Hkv, int S, int W, int kk, float scale, float sl2,
     float bl2, int combo, int tile, bf16_t *__restrict__ qc_ws, bf16_t *__restrict__ qr_ws,
     float *__restrict__ lse_ws, float *__restrict__ dd_ws, bf16_t *__restrict__ dq, float *__restrict__ dq_gain,
@@ -1364,20 +1368,18 @@ __device__ __forceinline__ void dq_body(
     uint32_t *qbits = reinterpret_cast<uint32_t *>(list + ((nb + 1) & ~1LL));
     uint32_t *wbits = qbits + QT * nbw;
 
-    // A ring slot: K tile [64][D] (swzK), V tile [64][D] (swzK), K^T tile
-    // [D][64] (swzV), in 1 KB parts; part w + WAVES*pp is this wave's.  The
+    // A ring slot: K tile and V tile, [64][D] (swzK), in 1 KB parts; part w + WAVES*pp is this wave's.  The
     // sources at block 0 and the stride per block are set once; a window tile
-    // reads kr / krt (the same rows of the other tensor) instead of kc / kct.
+    // reads kr (the same rows of the other tensor) instead of kc.
     const bf16_t *KC = kc + bh * n * D;
-    const bf16_t *KCT = kct + bh * D * n;
     const bf16_t *VB = v + ((int64_t)b * n * Hkv + g) * D;   // v [B, n, Hkv, D]
-    const int64_t dkr = kr - kc, dkrt = krt - kct;
+    const int64_t dkr = kr - kc;
     const bf16_t *dsrc[C::PPW];
     int64_t dstr[C::PPW], drot[C::PPW];
 #pragma unroll
     for (int pp = 0; pp < C::PPW; ++pp) {
         const int part = w + WAVES * pp;
-        const int tl = part / C::KPARTS;            // 0: K, 1: V, 2: K^T, 3: none
+        const int tl = part / C::KPARTS;            // 0: K, 1: V
         const int pc = (part % C::KPARTS) * 64 + lane;
         dsrc[pp] = KC;
         dstr[pp] = 0;
@@ -1391,11 +1393,6 @@ __device__ __forceinline__ void dq_body(
             const int r = pc / (D / 8), c = (pc % (D / 8)) ^ swzK(pc / (D / 8));
             dsrc[pp] = VB + (int64_t)r * Hkv * D + 8 * c;
             dstr[pp] = 64 * (int64_t)Hkv * D;
-        } else if (tl == 2) {
-            const int r = pc >> 3, c = (pc & 7) ^ swzV(pc >> 3);
-            dsrc[pp] = KCT + (int64_t)r * n + 8 * c;
-            dstr[pp] = 64;
-            drot[pp] = dkrt;
         }
     }
     const int dpw = (C::NPARTS - w + WAVES - 1) / WAVES;   // this wave's DMA instructions per block
@@ -1418,11 +1415,11 @@ __device__ __forceinline__ void dq_body(
     bf16x8 qop[PTW][NKS], dop[PTW][NKS];
     f32x4 acc[PTW][NDT];
     float mrun[PTW], lsum[PTW], Dh[PTW];
-    int64_t icol[PTW];
+    int icol[PTW];   // n / 64 fits 16 bits
     bool cok[PTW];
 #pragma unroll
     for (int t = 0; t < PTW; ++t) {
-        icol[t] = i0 + (int64_t)(w * PTW + t) * QPT + qs;
+        icol[t] = (int)i0 + (w * PTW + t) * QPT + qs;
         cok[t] = colv && icol[t] < n;
         mrun[t] = -INFINITY;
         lsum[t] = 0.0f;
@@ -1472,23 +1469,21 @@ __device__ __forceinline__ void dq_body(
 #pragma nounroll
         for (int e = e0; e < e1; ++e) {
             const bf16_t *Ks = ring + (e % NS) * C::SLOT;
-            const int64_t kb = (int64_t)(wt0 + e) * 64;
+            const int kb = (wt0 + e) * 64;
 #pragma unroll
             for (int tt = 0; tt < PTW; ++tt) {
-                const int64_t qa = i0 + (int64_t)(w * PTW + tt) * QPT;
+                const int qa = (int)i0 + (w * PTW + tt) * QPT;
                 if (qa >= n) break;
-                const int64_t qb = (qa + QPT - 1 < n) ? qa + QPT - 1 : n - 1;
-                const int64_t loa = ((int64_t)S > qa - W + 1) ? (int64_t)S : qa - W + 1;
-                const int64_t lob = ((int64_t)S > qb - W + 1) ? (int64_t)S : qb - W + 1;
+                const int qb = (int)min((int64_t)qa + QPT, n) - 1;
+                const int loa = max(S, qa - W + 1), lob = max(S, qb - W + 1);
                 if (kb > qb || kb + 63 < loa) continue;   // no column has a window key here
                 const bool full = kb >= lob && kb + 63 <= qa;
-                const int64_t lo = ((int64_t)S > icol[tt] - W + 1) ? (int64_t)S : icol[tt] - W + 1;
-                const int64_t jlo = lo - kb, jhi = cok[tt] ? icol[tt] - kb : -1;
+                const int jlo = max(S, icol[tt] - W + 1) - kb, jhi = cok[tt] ? icol[tt] - kb : -1;
                 // a full tile as the range 0..63 (one inlined copy of the update)
-                dq_update<D, FIXED, DQ_RANGE>(Ks, Ks + C::TILE, Ks + 2 * C::TILE, qop[tt], dop[tt], Dh[tt], acc[tt],
+                dq_update<D, FIXED, DQ_RANGE>(Ks, Ks + C::TILE, qop[tt], dop[tt], Dh[tt], acc[tt],
                                               mrun[tt], lsum[tt], true,
-                                              full ? 0 : (int)(jlo < 0 ? 0 : (jlo > 64 ? 64 : jlo)),
-                                              full ? 63 : (int)(jhi < -1 ? -1 : (jhi > 63 ? 63 : jhi)), sl2, bl2,
+                                              full ? 0 : min(max(jlo, 0), 64),
+                                              full ? 63 : min(max(jhi, -1), 63), sl2, bl2,
                                               l16, lg);
             }
         }
@@ -1502,7 +1497,12 @@ __device__ __forceinline__ void dq_body(
     for (int c = 0; c < ntot && c < NPRO; ++c) fill(sblk(c), c, false);
 #pragma unroll
     for (int t = 0; t < PTW; ++t) {
-        const int64_t ii = cok[t] ? icol[t] : 0;
+        int l16s = l16;   // opaque: the set-up's row addresses would live through the window tiles
+        asm volatile("" : "+v"(l16s));
+        const int isw = (int)i0 + (w * PTW + t) * QPT + l16s / G;
+        const bool okw = l16s < QPT * G && isw < n;
+        const int64_t ii = okw ? isw : 0;
+        const int h = g * G + l16s % G;
         // rope^T(z) = z cos + rot^T(z sin), rot^T([z1, z2]) = [z2, -z1]: element
         // d = 16 dt + 4 lg + e and its partner d ^ D/2 (dt ^ NDT/2) in this lane
         float cs[NDT][4], sn[NDT][4];
@@ -1533,7 +1533,7 @@ __device__ __forceinline__ void dq_body(
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
             const bf16x8 qv = ldb8(src + 32 * ks);
-            qop[t][ks] = cok[t] ? (FIXED ? scale8(qv, sl2) : qv) : bf16x8{};
+            qop[t][ks] = okw ? (FIXED ? scale8(qv, sl2) : qv) : bf16x8{};
         }
     }
 
@@ -1562,12 +1562,12 @@ __device__ __forceinline__ void dq_body(
                 const int c = c0 + j;
                 const bf16_t *Ks = ring + (c % NS) * C::SLOT;
                 if (c < hs) {   // keys j < S and j <= i
-                    const int64_t jh = (icol[tt] < (int64_t)S - 1) ? icol[tt] : (int64_t)S - 1;
-                    dq_update<D, FIXED, DQ_RANGE>(Ks, Ks + C::TILE, Ks + 2 * C::TILE, qop[tt], dop[tt], Dh[tt],
-                                                  acc[tt], mrun[tt], lsum[tt], true, 0, cok[tt] ? (int)jh : -1, sl2,
+                    const int jh = min(icol[tt], S - 1);
+                    dq_update<D, FIXED, DQ_RANGE>(Ks, Ks + C::TILE, qop[tt], dop[tt], Dh[tt],
+                                                  acc[tt], mrun[tt], lsum[tt], true, 0, cok[tt] ? jh : -1, sl2,
                                                   bl2, l16, lg);
                 } else {
-                    dq_update<D, FIXED, DQ_COL>(Ks, Ks + C::TILE, Ks + 2 * C::TILE, qop[tt], dop[tt], Dh[tt],
+                    dq_update<D, FIXED, DQ_COL>(Ks, Ks + C::TILE, qop[tt], dop[tt], Dh[tt],
                                                 acc[tt], mrun[tt], lsum[tt], (qw >> j) & 1u, 0, 63, sl2, bl2, l16, lg);
                 }
             }
@@ -1575,9 +1575,20 @@ __device__ __forceinline__ void dq_body(
     }
 
     // ------------- LSE, dq = QKNorm backward of scale * acc / l, gain sums
+    // The column's indexes once more, from the opaque thread index: kept from
+    // the set-up, their products with the strides would live (and spill)
+    // through the loops
     float gq[PTW];
+    int tide = tid;
+    asm volatile("" : "+v"(tide));
+    {
+    const int l16 = tide & 15, lg = (tide >> 4) & 3, qs = l16 / G, h = g * G + l16 % G;
+    int icol[PTW];
+    bool cok[PTW];
 #pragma unroll
     for (int t = 0; t < PTW; ++t) {
+        icol[t] = (int)i0 + (w * PTW + t) * QPT + qs;
+        cok[t] = l16 < QPT * G && icol[t] < n;
         float l = lsum[t];
         l += __shfl_xor(l, 16, 64);
         l += __shfl_xor(l, 32, 64);
@@ -1627,6 +1638,7 @@ __device__ __forceinline__ void dq_body(
             }
         }
     }
+    }
     if (qgain && dq_gain) {   // workgroup-uniform: per head over the workgroup's columns, one atomic each
         float *gs = reinterpret_cast<float *>(smem);   // the ring, once every wave is done with it: [WAVES * PTW][16]
         __syncthreads();
@@ -1646,9 +1658,8 @@ __device__ __forceinline__ void dq_body(
 template <int D, int WAVES, int PTW, int NS, int PH>
 __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void bwd_dq_union_kernel(
     const bf16_t *__restrict__ q, const float *__restrict__ qgain, const float *__restrict__ kgain, float eps,
-    const bf16_t *__restrict__ kc, const bf16_t *__restrict__ kr, const bf16_t *__restrict__ kct,
-    const bf16_t *__restrict__ krt, const bf16_t *__restrict__ v, const float *__restrict__ cosT,
-    const float *__restrict__ sinT, const int32_t *__restrict__ idx, const int32_t *__restrict__ cnt,
+    const bf16_t *__restrict__ kc, const bf16_t *__restrict__ kr, const bf16_t *__restrict__ v,
+    const float *__restrict__ cosT, const float *__restrict__ sinT, const int32_t *__restrict__ idx, const int32_t *__restrict__ cnt,
     const bf16_t *__restrict__ out, const bf16_t *__restrict__ dout, int64_t n, int Hq, int Hkv, int S, int W,
     int kk, float scale, int ntiles, int Cn, int xmap, bf16_t *__restrict__ qc_ws, bf16_t *__restrict__ qr_ws,
     float *__restrict__ lse_ws, float *__restrict__ dd_ws, bf16_t *__restrict__ dq, float *__restrict__ dq_gain) {
@@ -1661,11 +1672,11 @@ __global__ __launch_bounds__(WAVES * 64, WAVES / 4) void bwd_dq_union_kernel(
     const float sl2 = scale * LOG2E;
     float bl2;
     if (group_bound(qgain, kgain, combo % Hkv, G, sl2, D, bl2))
-        dq_body<D, WAVES, PTW, NS, PH, true>(q, qgain, eps, kc, kr, kct, krt, v, cosT, sinT, idx, cnt, out, dout, n,
+        dq_body<D, WAVES, PTW, NS, PH, true>(q, qgain, eps, kc, kr, v, cosT, sinT, idx, cnt, out, dout, n,
                                              Hq, Hkv, S, W, kk, scale, sl2, bl2, combo, tile, qc_ws, qr_ws, lse_ws,
                                              dd_ws, dq, dq_gain, smem, nlist);
     else
-        dq_body<D, WAVES, PTW, NS, PH, false>(q, qgain, eps, kc, kr, kct, krt, v, cosT, sinT, idx, cnt, out, dout,
+        dq_body<D, WAVES, PTW, NS, PH, false>(q, qgain, eps, kc, kr, v, cosT, sinT, idx, cnt, out, dout,
                                               n, Hq, Hkv, S, W, kk, scale, sl2, bl2, combo, tile, qc_ws, qr_ws,
                                               lse_ws, dd_ws, dq, dq_gain, smem, nlist);
 }
@@ -1771,7 +1782,7 @@ static size_t dq_lds(int64_t n, int64_t G, int64_t k) {
 
 template <int D, int WAVES, int PTW, int NS, int PH>
 static int launch_dq_t(const void *q, const float *qgain, const float *kgain, float eps, const void *kc,
-                       const void *kr, const void *kct, const void *krt, const void *v, const float *cosT,
+                       const void *kr, const void *v, const float *cosT,
                        const float *sinT, const int32_t *idx, const int32_t *cnt, const void *out, const void *dout,
                        int64_t B, int64_t n, int64_t Hq, int64_t Hkv, int64_t S, int64_t W, int64_t k, float scale,
                        void *qc_ws, void *qr_ws, float *lse_ws, float *dd_ws, void *dq, float *dq_gain,
@@ -1789,7 +1800,7 @@ static int launch_dq_t(const void *q, const float *qgain, const float *kgain, fl
                             (int)lds) != hipSuccess)
         return HBA_ERR_LAUNCH;
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(WAVES * 64), lds, s, (const bf16_t *)q, qgain, kgain, eps,
-                       (const bf16_t *)kc, (const bf16_t *)kr, (const bf16_t *)kct, (const bf16_t *)krt,
+                       (const bf16_t *)kc, (const bf16_t *)kr,
                        (const bf16_t *)v, cosT, sinT, idx, cnt, (const bf16_t *)out, (const bf16_t *)dout, n,
                        (int)Hq, (int)Hkv, (int)S, Wc, (int)k, scale, (int)ntiles, (int)(B * Hkv), xmap,
                        (bf16_t *)qc_ws, (bf16_t *)qr_ws, lse_ws, dd_ws, (bf16_t *)dq, dq_gain);
@@ -1838,7 +1849,7 @@ int launch_attn_bf16(const void *q, const int64_t *qs, const float *qgain, const
 
 template <int D>
 int launch_attn_bf16_dq(const void *q, const float *qgain, const float *kgain, float eps, const void *kc,
-                        const void *kr, const void *kct, const void *krt, const void *v, const float *cosT,
+                        const void *kr, const void *v, const float *cosT,
                         const float *sinT, const int32_t *idx, const int32_t *cnt, const void *out,
                         const void *dout, int64_t B, int64_t n, int64_t Hq, int64_t Hkv, int64_t S, int64_t W,
                         int64_t k, float scale, void *qc_ws, void *qr_ws, float *lse_ws, float *dd_ws, void *dq,
@@ -1848,23 +1859,23 @@ int launch_attn_bf16_dq(const void *q, const float *qgain, const float *kgain, f
     if (D != 64 || G > 16 || S > 64 || n % 64 || n / 64 >= SENT) return HBA_ERR_UNSUPPORTED;
     constexpr size_t LDS_MAX = 160 * 1024 - 64;   // 64 bytes for the static nlist
     // d = 64: 16 waves (4 per SIMD, within 128 VGPRs) of one row tile, 32
-    // queries at G = 7; a 6-slot ring (3 blocks per phase) when the selection
-    // lists fit beside it, else 4 slots.  Measured at 32K (whole backward):
-    // 16 x 1 3.74 ms, 12 waves x 2 tiles 4.11, 8 x 3 4.09 (2 waves per SIMD
-    // leave the update's LDS and MFMA latencies exposed); 16 x 1 with 2-block
-    // phases 4.00, with a 4-slot ring 3.90
-    if (dq_lds<64, 16, 1, 6>(n, G, k) <= LDS_MAX)
-        return launch_dq_t<64, 16, 1, 6, 3>(q, qgain, kgain, eps, kc, kr, kct, krt, v, cosT, sinT, idx, cnt, out,
-                                           dout, B, n, Hq, Hkv, S, W, k, scale, qc_ws, qr_ws, lse_ws, dd_ws, dq,
-                                           dq_gain, s);
+    // queries at G = 7; an 8-slot ring (4 blocks per phase) when the selection
+    // lists fit beside it, else 4 slots.  Measured at 32K, this kernel alone:
+    // 1.27 ms; 6 slots in two phases 1.39, 9 slots in three 1.48.  With K^T
+    // tiles staged beside K and V (24 KB per block) 6 slots took 1.42 ms, and
+    // the whole backward 3.74 ms against 4.11 for 12 waves x 2 tiles and 4.09
+    // for 8 x 3 (2 waves per SIMD leave the update's LDS and MFMA latencies
+    // exposed)
+    if (dq_lds<64, 16, 1, 8>(n, G, k) <= LDS_MAX)
+        return launch_dq_t<64, 16, 1, 8, 4>(q, qgain, kgain, eps, kc, kr, v, cosT, sinT, idx, cnt, out, dout, B, n, Hq,
+                                            Hkv, S, W, k, scale, qc_ws, qr_ws, lse_ws, dd_ws, dq, dq_gain, s);
     if (dq_lds<64, 16, 1, 4>(n, G, k) <= LDS_MAX)
-        return launch_dq_t<64, 16, 1, 4, 2>(q, qgain, kgain, eps, kc, kr, kct, krt, v, cosT, sinT, idx, cnt, out,
-                                           dout, B, n, Hq, Hkv, S, W, k, scale, qc_ws, qr_ws, lse_ws, dd_ws, dq,
-                                           dq_gain, s);
+        return launch_dq_t<64, 16, 1, 4, 2>(q, qgain, kgain, eps, kc, kr, v, cosT, sinT, idx, cnt, out, dout, B, n, Hq,
+                                            Hkv, S, W, k, scale, qc_ws, qr_ws, lse_ws, dd_ws, dq, dq_gain, s);
     return HBA_ERR_UNSUPPORTED;
 }
 template int launch_attn_bf16_dq<64>(const void *, const float *, const float *, float, const void *, const void *,
-                                     const void *, const void *, const void *, const float *, const float *,
+                                     const void *, const float *, const float *,
                                      const int32_t *, const int32_t *, const void *, const void *, int64_t, int64_t,
                                      int64_t, int64_t, int64_t, int64_t, int64_t, float, void *, void *, float *,
                                      float *, void *, float *, hipStream_t);

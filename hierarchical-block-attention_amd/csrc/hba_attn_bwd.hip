@@ -119,8 +119,8 @@ __device__ __forceinline__ float col_sum(float v) {
 constexpr int DKV_ROWS = 4096;
 constexpr int PB_WORDS = DKV_ROWS / 32;
 
-// transposed prepared keys, kct / krt [B, Hkv, d, n]: one workgroup per 64-key
-// tile; it also clears the tile's rows of the dk / dv accumulator dkv_acc
+// transposed prepared keys for bwd_dq_mfma, kct / krt [B, Hkv, d, n] (kct null:
+// none): one workgroup per 64-key tile; it also clears the tile's rows of the dk / dv accumulator dkv_acc
 // [B, Hkv, n, 3, d] (bwd_dkv_mfma adds into it next) and the tile's routed-row
 // bits of every range (bwd_pick_bits sets them next)
 template <int D>
@@ -138,6 +138,7 @@ __global__ __launch_bounds__(256) void bwd_kt_kernel(const bf16_t *__restrict__ 
         for (int e = threadIdx.x; e < nsplit * PB_WORDS; e += 256)
             pbits[((bg * nsplit + e / PB_WORDS) * nt + blk) * PB_WORDS + e % PB_WORDS] = 0u;
     }
+    if (!kct) return;
     for (int pass = 0; pass < 2; ++pass) {
         const bf16_t *src = (pass ? kr : kc) + (bg * n + kb) * D;
         bf16_t *dst = (pass ? krt : kct) + bg * D * n + kb;
@@ -539,19 +540,6 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dq_mfma_kernel(
 constexpr int SINK_ROWS = 256;   // query rows per workgroup of the sink launch
 constexpr int DKV_RL = 1024;   // routed rows run as one series of tiles at most
 constexpr int DKV_TP = 64;   // pairs per tile: two halves of 32, the pair count of one product
-
-// Elements 8 lg .. + 7 of a column of a row-major LDS tile: ds_read_b64_tr_b16
-// gives lane r of 16 the elements r % 4 of the four 8-byte pieces that lanes
-// r / 4 + 4 j (j = 0 .. 3) address, so lane r addresses columns 4 (r % 4) .. + 3
-// of row r / 4 (p0: of rows 0 .. 3, p1: of rows 4 .. 7) and receives column r.
-__device__ __forceinline__ bf16x8 ld_tr8(const bf16_t *p0, const bf16_t *p1) {
-    typedef short s16x4 __attribute__((ext_vector_type(4)));
-    typedef short s16x8 __attribute__((ext_vector_type(8)));
-    typedef __attribute__((address_space(3))) s16x4 *lds4;
-    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)p0);
-    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)p1);
-    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
-}
 
 __device__ __forceinline__ int pslot(int mt, int r) { return 8 * (r >> 2) + 4 * mt + (r & 3); }
 
@@ -1045,25 +1033,25 @@ extern "C" int hba_attn_bwd(int dtype, const void *q, const void *k, const void 
     if (g3 > 0x7fffffffLL) return HBA_ERR_UNSUPPORTED;
 #define HBA_BWD(D)                                                                                              \
     do {                                                                                                        \
-        hipLaunchKernelGGL((bw::bwd_kt_kernel<D>), dim3((unsigned)g2), dim3(256), 0, s, (const bf16_t *)kc,      \
-                           (const bf16_t *)kr, kct, krt, n, dkv_acc, pbits, nsplit_kv);                          \
-        hipLaunchKernelGGL(bw::bwd_pick_bits_kernel, dim3((unsigned)gpb), dim3(256), 0, s, idx, cnt, n, n / 64,  \
-                           (int)k_blocks, B * Hkv * n * k_blocks, nsplit_kv, pbits);                             \
         int dqs = HBA_ERR_UNSUPPORTED;                                                                          \
         if constexpr (D == 64)                                                                                  \
             if (bwd_dq_union_on())                                                                              \
-                dqs = launch_attn_bf16_dq<D>(q, q_gain, k_gain, eps, kc, kr, kct, krt, v, cos_tab, sin_tab,      \
+                dqs = launch_attn_bf16_dq<D>(q, q_gain, k_gain, eps, kc, kr, v, cos_tab, sin_tab,                \
                                              idx, cnt, out, dout, B, n, Hq, Hkv, S, W, k_blocks, scale,          \
                                              qcb_ws, qrb_ws, lse_ws, dd_ws, dq, dq_gain, s);                     \
-        if (dqs == HBA_ERR_UNSUPPORTED)                                                                         \
+        if (dqs != HBA_OK && dqs != HBA_ERR_UNSUPPORTED) return dqs;                                            \
+        const bool kt = dqs != HBA_OK;                                                                          \
+        hipLaunchKernelGGL((bw::bwd_kt_kernel<D>), dim3((unsigned)g2), dim3(256), 0, s, (const bf16_t *)kc,      \
+                           (const bf16_t *)kr, kt ? kct : nullptr, krt, n, dkv_acc, pbits, nsplit_kv);           \
+        hipLaunchKernelGGL(bw::bwd_pick_bits_kernel, dim3((unsigned)gpb), dim3(256), 0, s, idx, cnt, n, n / 64,  \
+                           (int)k_blocks, B * Hkv * n * k_blocks, nsplit_kv, pbits);                             \
+        if (kt)                                                                                                 \
             hipLaunchKernelGGL((bw::bwd_dq_mfma_kernel<D>), dim3((unsigned)g1q), dim3(256), 0, s,                \
                                (const bf16_t *)q, (const bf16_t *)kc, (const bf16_t *)kr, kct, krt,             \
                                (const bf16_t *)v, q_gain, eps, cos_tab, sin_tab, idx, cnt,                      \
                                (const bf16_t *)out, (const bf16_t *)dout, (int)B, n, (int)Hq, (int)Hkv,         \
                                (int)S, W, (int)k_blocks, scale, qpw, qcb_ws, qrb_ws, lse_ws, dd_ws,             \
                                (bf16_t *)dq, dq_gain);                                                          \
-        else if (dqs != HBA_OK)                                                                                 \
-            return dqs;                                                                                         \
         if (S > 0)                                                                                              \
             hipLaunchKernelGGL((bw::bwd_dkv_mfma_kernel<D>), dim3((unsigned)gs), dim3(bw::DKV_NT), 0, s,         \
                                (const bf16_t *)kc, (const bf16_t *)kr, (const bf16_t *)v, idx, cnt,              \

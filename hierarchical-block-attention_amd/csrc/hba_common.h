@@ -159,6 +159,19 @@ __device__ __forceinline__ float div_rn_fast(float x, float r, float inv) {
     return (e == 0.0f) ? q0 : fmaf(e, inv, q0);
 }
 
+// Elements 8 lg .. + 7 of a column of a row-major LDS tile: ds_read_b64_tr_b16
+// gives lane r of 16 the elements r % 4 of the four 8-byte pieces that lanes
+// r / 4 + 4 j (j = 0 .. 3) address, so lane r addresses columns 4 (r % 4) .. + 3
+// of row r / 4 (p0: of rows 0 .. 3, p1: of rows 4 .. 7) and receives column r.
+__device__ __forceinline__ bf16x8 ld_tr8(const bf16_t *p0, const bf16_t *p1) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    typedef __attribute__((address_space(3))) s16x4 *lds4;
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)p0);
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)p1);
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
 // ----------------------------------------------------------- wave helpers --
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
