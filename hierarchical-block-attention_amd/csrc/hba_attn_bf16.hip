@@ -1752,7 +1752,10 @@ static int launch_routed_t(const void *q, const int64_t *qs, const float *qgain,
     return (S > 64) ? go(&attn_routed_kernel<D, PTW, true, WIN>) : go(&attn_routed_kernel<D, PTW, false, WIN>);
 }
 
-// PTW row tiles per wave when the selection lists fit LDS beside the ring, else one
+// PTW row tiles per wave when the selection lists fit LDS beside the ring, else
+// one.  One also where twice the workgroups still find a compute unit each
+// (one fills its LDS): each column sums its blocks in the same order either way.
+constexpr int64_t CUS = 256;
 template <int D, bool WIN>
 static int launch_routed(const void *q, const int64_t *qs, const float *qgain, const float *kgain, float eps,
                          const void *kc, const void *vt, const int32_t *idx, const int32_t *cnt, int64_t B,
@@ -1761,7 +1764,9 @@ static int launch_routed(const void *q, const int64_t *qs, const float *qgain, c
                          int64_t W, void *qrw, hipStream_t s) {
     constexpr size_t LDS_MAX = 160 * 1024 - 64;   // 64 bytes for the static nlist
     const int64_t G = Hq / Hkv;
-    if (routed_lds<D, RtCfg<D>::PTW>(n, G, k) <= LDS_MAX)
+    const int64_t QT = (int64_t)RtCfg<D>::WAVES * RtCfg<D>::PTW * (16 / G);
+    const bool wide = RtCfg<D>::PTW == 1 || B * Hkv * ((n + QT - 1) / QT) > CUS / 2;
+    if (wide && routed_lds<D, RtCfg<D>::PTW>(n, G, k) <= LDS_MAX)
         return launch_routed_t<D, RtCfg<D>::PTW, WIN>(q, qs, qgain, kgain, eps, kc, vt, idx, cnt, B, n, Hq, Hkv, S,
                                                        k, scale, out, os, lse, kr, cosT, sinT, W, qrw, s);
     if (RtCfg<D>::PTW > 1 && routed_lds<D, 1>(n, G, k) <= LDS_MAX)

@@ -1342,6 +1342,19 @@ __global__ __launch_bounds__(256, 2) void score_select_thr_kernel(
     sel_deep_first(ntiles, Hkv, tile, g, b);
     const int G = Hq / Hkv;
     const int64_t i0 = (int64_t)tile * QW;
+    const int64_t last = (i0 + QW - 1 < n) ? i0 + QW - 1 : n - 1;
+    const int tile_bmax = (int)cand_bmax(last, 64, W);
+    if (tile_bmax < 1) {   // no query of the tile has a candidate
+        for (int e = tid; e < QW * kk; e += 256) {
+            const int64_t iq = i0 + e / kk;
+            if (iq >= n) break;
+            const int64_t o = ((b * Hkv + g) * n + i0) * kk + e;
+            idx[o] = -1;
+            val[o] = -INFINITY;
+        }
+        if (tid < QW && i0 + tid < n) cnt[(b * Hkv + g) * n + i0 + tid] = 0;
+        return;
+    }
     routing_queries_tile<D, ROWQ>(q, qsb, qsn, qsh, qgain, eps, b, i0, n, g, G, qgs, tid);
     __syncthreads();
     bf16x8 qb[NCT][NKS];
@@ -1354,8 +1367,6 @@ __global__ __launch_bounds__(256, 2) void score_select_thr_kernel(
         const int64_t iq = i0 + qc;
         bmax[ct] = (iq < n) ? (int)cand_bmax(iq, 64, W) : 0;
     }
-    const int64_t last = (i0 + QW - 1 < n) ? i0 + QW - 1 : n - 1;
-    const int tile_bmax = (int)cand_bmax(last, 64, W);
     // every query of the tile has the candidates 1 .. bmin (bmax grows with i)
     const int bmin = (i0 + QW - 1 < n) ? (int)cand_bmax(i0, 64, W) : 0;
     const int nst = (tile_bmax > 0) ? (tile_bmax + CB - 1) / CB : 0;
