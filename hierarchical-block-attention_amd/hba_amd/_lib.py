@@ -96,6 +96,9 @@ def check(status, what):
         raise HBAError(f"{what}: {msg} (status {status})")
 
 
+_I64X3 = ctypes.c_int64 * 3
+
+
 def strides3(t):
     """First three strides (elements) of a 4-D [B, n, H, d] view as a ctypes array."""
-    return (ctypes.c_int64 * 3)(*[int(s) for s in t.stride()[:3]])
+    return _I64X3(*t.stride()[:3])
