@@ -553,20 +553,30 @@ __global__ __launch_bounds__(256, 3) void attn_win_kernel(
     const bf16_t *__restrict__ q, int64_t qsb, int64_t qsn, int64_t qsh, const float *__restrict__ qgain,
     const float *__restrict__ kgain, float eps, const bf16_t *__restrict__ kr, const bf16_t *__restrict__ vt,
     const float *__restrict__ cosT, const float *__restrict__ sinT, int n, int Hq, int Hkv, int S,
-    int W, float scale, int gw, int hsplit, int wsplit, int ntiles, int Cn,
+    int W, float scale, int gw, int hsplit, int wsplit, int ntiles, int Cn, int xmap,
     bf16_t *__restrict__ out, int64_t osb, int64_t osn, int64_t osh, float *__restrict__ lse) {
     extern __shared__ __align__(16) char smem[];
-    // Work unit u = ((combo * ntiles + tile) * hsplit + hs), hs fastest.  XCD
-    // x (workgroup i runs on XCD i % 8) takes the x-th contiguous eighth of
-    // the units, so the heads and neighbouring tiles that read the same
-    // keys share that XCD's L2.
-    const int U = Cn * ntiles;
-    const int chunk = (U + 7) / 8;
-    const int u = (int)(blockIdx.x & 7) * chunk + (int)(blockIdx.x >> 3);
-    if (u >= U) return;
-    const int hs = u % hsplit;
-    const int tile = (u / hsplit) % ntiles;
-    const int combo = u / (hsplit * ntiles);
+    int hs, tile, combo;
+    if (xmap < 0) {
+        // Work unit u = ((combo * ntiles + tile) * hsplit + hs), hs fastest.
+        // XCD x (workgroup i runs on XCD i % 8) takes the x-th contiguous
+        // eighth of the units, so the heads and neighbouring tiles that read
+        // the same keys share that XCD's L2.
+        const int U = Cn * ntiles;
+        const int chunk = (U + 7) / 8;
+        const int u = (int)(blockIdx.x & 7) * chunk + (int)(blockIdx.x >> 3);
+        if (u >= U) return;
+        hs = u % hsplit;
+        tile = (u / hsplit) % ntiles;
+        combo = u / (hsplit * ntiles);
+    } else {
+        // a window past half of the sequence: deepest tiles first (launch_win)
+        int u;
+        xcd_map(blockIdx.x, Cn / hsplit, ntiles * hsplit, xmap, combo, u);
+        if (u >= ntiles * hsplit || combo >= Cn / hsplit) return;
+        hs = u % hsplit;
+        tile = u / hsplit;
+    }
     const int G = Hq / Hkv;
     const float sl2 = scale * LOG2E;
     float bl2;
@@ -1700,7 +1710,14 @@ static int launch_win(const void *q, const int64_t *qs, const float *qgain, cons
     const int64_t ntiles = (n + QT - 1) / QT;
     const int64_t Cn = B * Hkv * hsplit;
     const int64_t U = Cn * ntiles;
-    const int64_t grid = 8 * ((U + 7) / 8);
+    // Tiles of a window that covers more than half of the sequence grow with
+    // their position, and an eighth of the units per XCD gives some XCDs the
+    // deepest tiles only: deepest first over all of them instead.  Dense
+    // causal attention of 8128 tokens, 14 / 2 heads, head dim 64: 310 us in
+    // eighths, 183 deepest first (943 against 1313 for 8192 tokens, 28 / 4 heads, head dim 128).  Tiles of a shorter window cost alike,
+    // and stay next to the tiles that read the same keys.
+    int64_t grid = 8 * ((U + 7) / 8);
+    const int xmap = 2 * W > n ? xcd_pick(B * Hkv, ntiles * hsplit, grid) : -1;
     if (grid > 0x7fffffff) return HBA_ERR_UNSUPPORTED;
     const size_t lds = (size_t)C::NS * C::SLOT * 2;
     if (hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_win_kernel<D, RT>),
@@ -1709,7 +1726,7 @@ static int launch_win(const void *q, const int64_t *qs, const float *qgain, cons
     const int Wc = (int)((W < n + 1) ? W : n + 1);     // a window longer than the sequence is the sequence
     hipLaunchKernelGGL((attn_win_kernel<D, RT>), dim3((unsigned)grid), dim3(nthr), lds, s, (const bf16_t *)q, qs[0],
                        qs[1], qs[2], qgain, kgain, eps, (const bf16_t *)kr, (const bf16_t *)vt, cosT, sinT, (int)n,
-                       (int)Hq, (int)Hkv, (int)S, Wc, scale, gw, hsplit, wsplit, (int)ntiles, (int)Cn,
+                       (int)Hq, (int)Hkv, (int)S, Wc, scale, gw, hsplit, wsplit, (int)ntiles, (int)Cn, xmap,
                        (bf16_t *)out, os[0], os[1], os[2], lse);
     return HBA_OK;
 }
@@ -1753,8 +1770,11 @@ static int launch_routed_t(const void *q, const int64_t *qs, const float *qgain,
 }
 
 // PTW row tiles per wave when the selection lists fit LDS beside the ring, else
-// one.  One also where twice the workgroups still find a compute unit each
-// (one fills its LDS): each column sums its blocks in the same order either way.
+// one.  One also where two would leave no more than a workgroup per compute
+// unit (each column sums its blocks in the same order either way).  14 / 2
+// heads, d = 64, two tiles against one: 1216 tokens (38 workgroups of two) 54.6
+// and 32.0 us, 4096 (128) 116 and 70, 6144 (192) 131 and 107, 8192 (256) 146
+// and 143, 16384 (512) 301 and 337.
 constexpr int64_t CUS = 256;
 template <int D, bool WIN>
 static int launch_routed(const void *q, const int64_t *qs, const float *qgain, const float *kgain, float eps,
@@ -1765,7 +1785,7 @@ static int launch_routed(const void *q, const int64_t *qs, const float *qgain, c
     constexpr size_t LDS_MAX = 160 * 1024 - 64;   // 64 bytes for the static nlist
     const int64_t G = Hq / Hkv;
     const int64_t QT = (int64_t)RtCfg<D>::WAVES * RtCfg<D>::PTW * (16 / G);
-    const bool wide = RtCfg<D>::PTW == 1 || B * Hkv * ((n + QT - 1) / QT) > CUS / 2;
+    const bool wide = RtCfg<D>::PTW == 1 || B * Hkv * ((n + QT - 1) / QT) > CUS;
     if (wide && routed_lds<D, RtCfg<D>::PTW>(n, G, k) <= LDS_MAX)
         return launch_routed_t<D, RtCfg<D>::PTW, WIN>(q, qs, qgain, kgain, eps, kc, vt, idx, cnt, B, n, Hq, Hkv, S,
                                                        k, scale, out, os, lse, kr, cosT, sinT, W, qrw, s);
