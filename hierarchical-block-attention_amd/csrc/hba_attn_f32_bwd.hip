@@ -284,10 +284,11 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dq_f32_kernel(
 
 // Workgroup (b, g, range of R query rows, 64-key block); the block index nb
 // stands for the sink keys of block 0, which every row from j on attends.
-// 256-row ranges give a 2048-token call (32 blocks, 2 KV heads) about 400
-// workgroups with a window's rows; longer sequences take longer ranges, so
-// that a (range, block) pair does not run for a handful of routed rows.
-constexpr int F32_RMIN = 256, F32_RMAX = 2048;
+// About 32 ranges per sequence balance the blocks' rows (a block that many
+// queries picked, a range that a window only touches): at 2048 tokens, 14 / 2
+// heads, ranges of 256 rows took 424 us, 128 303, 64 263; at 4096 256 853, 128
+// 790.  Past 64K tokens ranges stay at 2048 rows, so that the list fits LDS.
+constexpr int F32_RMIN = 64, F32_RMAX = 2048;
 
 template <int D>
 __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dkv_f32_kernel(
@@ -540,7 +541,7 @@ int launch_attn_bwd_f32(const float *q, const float *k, const float *v, const fl
     int64_t grid;
     const int xmap = xcd_pick(Cn, ntiles, grid);
     int64_t R = af::F32_RMIN;
-    while (n / R > 16 && R < af::F32_RMAX) R *= 2;
+    while (n / R > 32 && R < af::F32_RMAX) R *= 2;
     const int64_t nsplit = (n + R - 1) / R, nblk = n / 64 + (S > 0), grid2 = Cn * nsplit * nblk;
     if (grid > 0x7fffffffLL || grid2 > 0x7fffffffLL || n > 0x3fffffffLL || n * Hq > 0x7fffffffLL)
         return HBA_ERR_UNSUPPORTED;
