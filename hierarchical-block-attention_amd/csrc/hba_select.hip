@@ -10,6 +10,8 @@
 // (score descending, block index ascending).
 #include <type_traits>
 
+#include <algorithm>
+
 #include "hba_common.h"
 #include "hba_abi.h"
 #include "hba_generic.h"
@@ -156,6 +158,152 @@ __device__ __forceinline__ void stage_blocks(float *lds, const typename St<DT>::
     const int total = cnt * M * D;
     const typename St<DT>::T *src = S + first * M * D;
     for (int e = threadIdx.x; e < total; e += SEL_WG) lds[e] = St<DT>::ld(src, e);
+}
+
+// (score, block) as one unsigned key ordered like (score desc, block asc):
+// the score's bits mapped to an order-preserving unsigned (a zero score
+// taken as +0, which the float comparison treats as equal to -0), then the
+// complement of the block.
+__device__ __forceinline__ uint64_t sel_key(float v, int blk) {
+    const uint32_t u = __float_as_uint(v + 0.0f);
+    const uint32_t ord = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+    return ((uint64_t)ord << 32) | (uint32_t)(0xffffffffu - (uint32_t)blk);
+}
+__device__ __forceinline__ float sel_key_score(uint64_t key) {
+    const uint32_t ord = (uint32_t)(key >> 32);
+    return __uint_as_float((ord & 0x80000000u) ? (ord & 0x7fffffffu) : ~ord);
+}
+__device__ __forceinline__ int sel_key_block(uint64_t key) { return (int)(0xffffffffu - (uint32_t)key); }
+
+// ---------------------------------------------------- flat top-k in fp32 ----
+// A workgroup takes 64 queries of one KV head, lane = query; its NW waves
+// share the candidate blocks (wave w takes 1 + w, 1 + w + NW, ...), keep a
+// sorted list each, and rank their entries against the other lists.  The
+// arithmetic and the order are score_select_kernel's: the heads are added in
+// order, every score is one chain over d, ties go to the lower block.  The
+// summaries are wave-uniform, so they come as scalar operands.  Bound by the
+// latency of its phases; with one wave per 64 queries (the LDS-staged kernel
+// below) a 4096-token call of 14 / 2 heads, head dim 64, had 128 waves on the
+// chip and took 115 us, this one 46.
+template <int KMAX>
+constexpr int flat_waves() {   // the lists fill 64 KB of LDS
+    return KMAX <= 16 ? 8 : 4;
+}
+
+template <int D, int M, int KMAX>
+__global__ __launch_bounds__(64 * flat_waves<KMAX>()) void score_select_f32_kernel(
+    const float *__restrict__ q, int64_t qsb, int64_t qsn, int64_t qsh, const float *__restrict__ qgain, float eps,
+    const float *__restrict__ S0, int64_t n, int Hq, int Hkv, int64_t nb, int64_t W, int kk, float scale,
+    int32_t *__restrict__ idx, float *__restrict__ val, int32_t *__restrict__ cnt, float *__restrict__ scores) {
+    constexpr int NW = flat_waves<KMAX>();
+    constexpr size_t UB = std::max((size_t)NW * KMAX * 64 * 8, (size_t)D * 64 * 4);
+    __shared__ __align__(16) char pool[UB];
+    __shared__ int counts[NW][64];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = blockIdx.y, G = Hq / Hkv;
+    const int64_t b = blockIdx.z;
+    const int64_t i0 = (int64_t)(gridDim.x - 1 - blockIdx.x) * 64;   // the most candidates first
+    const int64_t i = i0 + lane;                                     // n is a multiple of 64
+    const int bmax = (int)cand_bmax(i, 64, W), tile_bmax = (int)cand_bmax(i0 + 63, 64, W);
+    float vals[KMAX];
+    int ids[KMAX];
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) {
+        vals[j] = -INFINITY;
+        ids[j] = -1;
+    }
+    if (tile_bmax >= 1) {
+        // the routing queries: a wave prepares one head's rows, the heads are
+        // added in order
+        float *qs = reinterpret_cast<float *>(pool);   // [D][64]
+        float x[D];
+        for (int h0 = 0; h0 < G; h0 += NW) {
+            if (h0 + w < G) {
+                const int h = g * G + h0 + w;
+                const float4 *row = reinterpret_cast<const float4 *>(q + b * qsb + i * qsn + (int64_t)h * qsh);
+#pragma unroll
+                for (int c = 0; c < D / 4; ++c) {
+                    const float4 u = row[c];
+                    x[4 * c] = u.x;
+                    x[4 * c + 1] = u.y;
+                    x[4 * c + 2] = u.z;
+                    x[4 * c + 3] = u.w;
+                }
+                if (qgain) qknorm_row<0, D>(x, qgain[h], eps);
+            }
+            for (int s = 0; s < NW && h0 + s < G; ++s) {
+                if (w == s) {
+#pragma unroll
+                    for (int t = 0; t < D; ++t) qs[t * 64 + lane] = (h0 + s == 0) ? x[t] : qs[t * 64 + lane] + x[t];
+                }
+                __syncthreads();
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < D; ++t) x[t] = qs[t * 64 + lane];
+        __syncthreads();   // the lists take its place
+        const float *Sg = S0 + (b * Hkv + g) * nb * M * D;
+        for (int blk = 1 + w; blk <= tile_bmax; blk += NW) {
+            const float *S = Sg + (int64_t)blk * M * D;
+            float acc[M];
+#pragma unroll
+            for (int s = 0; s < M; ++s) acc[s] = 0.0f;
+#pragma unroll
+            for (int t = 0; t < D; ++t)
+#pragma unroll
+                for (int s = 0; s < M; ++s) acc[s] = fmaf(x[t], S[s * D + t], acc[s]);
+            float best = acc[0];
+#pragma unroll
+            for (int s = 1; s < M; ++s) best = (acc[s] > best) ? acc[s] : best;
+            const float v = best * scale;
+            if (blk <= bmax) {
+                if (scores) scores[((b * Hkv + g) * n + i) * nb + blk] = v;
+                insert_inorder<KMAX>(vals, ids, v, blk);
+            }
+        }
+    }
+    // the lists as keys that order as (score desc, block asc); 0: no entry
+    uint64_t *keys = reinterpret_cast<uint64_t *>(pool);   // [NW][KMAX][64]
+    uint64_t own[KMAX];
+    int rank[KMAX], c = 0;
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) {
+        own[j] = (vals[j] != -INFINITY) ? sel_key(vals[j], ids[j]) : 0ull;
+        c += own[j] != 0ull;
+        rank[j] = j;
+        keys[(w * KMAX + j) * 64 + lane] = own[j];
+    }
+    counts[w][lane] = c;
+    __syncthreads();
+    int total = 0;
+    for (int u = 0; u < NW; ++u) {
+        total += counts[u][lane];
+        if (u == w) continue;
+        const uint64_t *other = keys + u * KMAX * 64 + lane;
+        int p = 0;
+        uint64_t key = other[0];
+#pragma unroll
+        for (int j = 0; j < KMAX; ++j) {   // both lists descend
+            while (key > own[j]) {
+                ++p;
+                key = (p < KMAX) ? other[p * 64] : 0ull;
+            }
+            rank[j] += p;
+        }
+    }
+    const int64_t o = ((b * Hkv + g) * n + i) * kk;
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j)
+        if (own[j] != 0ull && rank[j] < kk) {
+            idx[o + rank[j]] = ids[j];
+            val[o + rank[j]] = vals[j];
+        }
+    for (int j = total + w; j < kk; j += NW) {
+        idx[o + j] = -1;
+        val[o + j] = -INFINITY;
+    }
+    if (w == 0) cnt[(b * Hkv + g) * n + i] = min(total, kk);
 }
 
 template <int DT, int D, int M, int KMAX>
@@ -426,20 +574,6 @@ __device__ __forceinline__ void routing_queries_tile(const bf16_t *q, int64_t qs
 // then inserts only children of those supers.  On a GPU tile of 64 queries
 // the kept supers cover nearly every super, so the children are scored as the
 // flat GEMM and filtered, not gathered.
-// (score, block) as one unsigned key ordered like (score desc, block asc):
-// the score's bits mapped to an order-preserving unsigned (a zero score
-// taken as +0, which the float comparison treats as equal to -0), then the
-// complement of the block.
-__device__ __forceinline__ uint64_t sel_key(float v, int blk) {
-    const uint32_t u = __float_as_uint(v + 0.0f);
-    const uint32_t ord = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-    return ((uint64_t)ord << 32) | (uint32_t)(0xffffffffu - (uint32_t)blk);
-}
-__device__ __forceinline__ float sel_key_score(uint64_t key) {
-    const uint32_t ord = (uint32_t)(key >> 32);
-    return __uint_as_float((ord & 0x80000000u) ? (ord & 0x7fffffffu) : ~ord);
-}
-__device__ __forceinline__ int sel_key_block(uint64_t key) { return (int)(0xffffffffu - (uint32_t)key); }
 
 // Position of the r-th (0-based) set bit of m; m must hold more than r.
 __device__ __forceinline__ int nth_set_bit64(uint64_t m, int r) {
@@ -1672,10 +1806,16 @@ void launch_flat(const void *q, const int64_t *qs, const float *qgain, float eps
             return;
         }
     }
-    hipLaunchKernelGGL((score_select_kernel<DT, D, M, KMAX>), grid, dim3(SEL_WG), 0, s,
-                       (const typename St<DT>::T *)q, qs[0], qs[1], qs[2], qgain, eps,
-                       (const typename St<DT>::T *)S0, n, (int)Hq, (int)Hkv, n / 64, W, (int)k,
-                       scale, idx, val, cnt, scores);
+    // (64-entry lists and their ranks do not fit a lane's registers)
+    if constexpr (DT == 0 && KMAX <= 32)
+        hipLaunchKernelGGL((score_select_f32_kernel<D, M, KMAX>), grid, dim3(64 * flat_waves<KMAX>()), 0, s,
+                           (const float *)q, qs[0], qs[1], qs[2], qgain, eps, (const float *)S0, n, (int)Hq, (int)Hkv,
+                           n / 64, W, (int)k, scale, idx, val, cnt, scores);
+    else
+        hipLaunchKernelGGL((score_select_kernel<DT, D, M, KMAX>), grid, dim3(SEL_WG), 0, s,
+                           (const typename St<DT>::T *)q, qs[0], qs[1], qs[2], qgain, eps,
+                           (const typename St<DT>::T *)S0, n, (int)Hq, (int)Hkv, n / 64, W, (int)k,
+                           scale, idx, val, cnt, scores);
 }
 
 // Workspace of the grouped level 2 (hier_l2_kernel): the routing queries
