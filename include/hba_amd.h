@@ -466,8 +466,7 @@ int hba_attn_bwd(int dtype, const void *q, const void *k, const void *v,
 
 /* Scratch bytes hba_attn_bwd needs for this dtype and Hkv: the QKNorm'd and
  * rotated query rows (2*B*n*Hq*d in the storage type), the per-row LSE and
- * <dout, out> (2*B*Hq*n fp32), the sink-key accumulators (2*B*Hkv*64*d
- * fp32); on the bf16 path also the transposed prepared keys (2*B*Hkv*n*d
+ * <dout, out> (2*B*Hq*n fp32), an unused 2*B*Hkv*64*d fp32; on the bf16 path also the transposed prepared keys (2*B*Hkv*n*d
  * bf16), the dk/dv accumulators (3*B*Hkv*n*d fp32) and the routed-row bits
  * (B*Hkv*ceil(n/4096)*(n/64)*512 bytes: one bit per query row of each
  * 4096-row range and key block); each part rounded up to 256 bytes. */
