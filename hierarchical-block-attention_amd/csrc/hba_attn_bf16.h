@@ -28,8 +28,8 @@ int launch_attn_bf16_routed(const void *q, const int64_t *qs, const float *qgain
                             int64_t n, int64_t Hq, int64_t Hkv, int64_t S, int64_t k, float scale, void *out,
                             const int64_t *os, const float *lse, hipStream_t s);
 
-// The query gradient of the union attention (bf16, d = 64, G <= 16, S <= 64;
-// HBA_ERR_UNSUPPORTED otherwise): dq (raw q) and the gain gradient added into
+// The query gradient of the union attention (bf16, G <= 16, S <= 64, selection
+// lists that fit LDS; HBA_ERR_UNSUPPORTED otherwise): dq (raw q) and the gain gradient added into
 // dq_gain, and for the key gradients the QKNorm'd and rotated rows (qc_ws,
 // qr_ws: bf16 [B, n, Hq, D]), the LSE and D (lse_ws, dd_ws: fp32 [B, Hq, n]).
 // v, out, dout as the forward's inputs and output.

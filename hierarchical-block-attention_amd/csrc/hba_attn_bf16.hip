@@ -1224,6 +1224,9 @@ struct DqCfg {
     static constexpr int NKS = D / 32;
     static constexpr int NDT = D / 16;
     static constexpr int NTHR = WAVES * 64;
+    // d = 64: the fixed shift's query operand carries scale * log2(e), rounded
+    // to bf16; d = 128: an fma per score instead, as exact as a running max
+    static constexpr bool FOLD = D == 64;
     static constexpr int TILE = 64 * D;                   // bf16 elements of a K or V tile
     static constexpr int SLOT = 2 * TILE;
     static constexpr int KPARTS = TILE * 2 / 1024;        // 1 KB parts of a tile
@@ -1256,7 +1259,9 @@ __device__ __forceinline__ void dq_update(const bf16_t *Ks, const bf16_t *Vk, co
     constexpr int NKS = D / 32, NDT = D / 16;
     asm volatile("" ::: "memory");   // no fragment held over from the previous row tile
     const bool cdead = MODE == DQ_COL && !colok;
-    const float c0 = FIXED ? (cdead ? -INFINITY : -bl2) : 0.0f;
+    constexpr bool FOLD = FIXED && DqCfg<D, 8>::FOLD;
+    const float c0 = FOLD ? (cdead ? -INFINITY : -bl2) : 0.0f;
+    const float sh0 = cdead ? INFINITY : bl2;   // FIXED without FOLD: a dead column's arguments are -inf
     const int sw = swzK(permk(0, l16));   // the same for every mt
     f32x4 Sa[4];
 #pragma unroll
@@ -1274,7 +1279,7 @@ __device__ __forceinline__ void dq_update(const bf16_t *Ks, const bf16_t *Vk, co
             for (int e = 0; e < 4; ++e) {
                 const int j = 32 * (mt >> 1) + 8 * lg + 4 * (mt & 1) + e;
                 const bool ok = (MODE != DQ_RANGE) || ((j >= jlo) & (j <= jhi));
-                p[mt][e] = ex2(ok ? Sa[mt][e] : -INFINITY);
+                p[mt][e] = ex2(ok ? (FOLD ? Sa[mt][e] : fmaf(Sa[mt][e], sl2, -sh0)) : -INFINITY);
             }
     } else {
         float tmax = -INFINITY;
@@ -1448,7 +1453,7 @@ __device__ __forceinline__ void dq_body(
                 *reinterpret_cast<u32x4 *>(qc_ws + row + 32 * ks) = __builtin_bit_cast(u32x4, qn[ks]);
                 *reinterpret_cast<u32x4 *>(qr_ws + row + 32 * ks) = __builtin_bit_cast(u32x4, qr[ks]);
             }
-            qop[t][ks] = FIXED ? scale8(qr[ks], sl2) : qr[ks];
+            qop[t][ks] = FIXED && C::FOLD ? scale8(qr[ks], sl2) : qr[ks];
             const u32x4 du = *reinterpret_cast<const u32x4 *>(dout + row + 32 * ks);
             const u32x4 uo = *reinterpret_cast<const u32x4 *>(out + row + 32 * ks);
             dop[t][ks] = cok[t] ? __builtin_bit_cast(bf16x8, du) : bf16x8{};
@@ -1543,7 +1548,7 @@ __device__ __forceinline__ void dq_body(
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
             const bf16x8 qv = ldb8(src + 32 * ks);
-            qop[t][ks] = okw ? (FIXED ? scale8(qv, sl2) : qv) : bf16x8{};
+            qop[t][ks] = okw ? (FIXED && C::FOLD ? scale8(qv, sl2) : qv) : bf16x8{};
         }
     }
 
@@ -1881,8 +1886,18 @@ int launch_attn_bf16_dq(const void *q, const float *qgain, const float *kgain, f
                         float *dq_gain, hipStream_t s) {
     using namespace ab;
     const int64_t G = Hq / Hkv;
-    if (D != 64 || G > 16 || S > 64 || n % 64 || n / 64 >= SENT) return HBA_ERR_UNSUPPORTED;
+    if (G > 16 || S > 64 || n % 64 || n / 64 >= SENT) return HBA_ERR_UNSUPPORTED;
     constexpr size_t LDS_MAX = 160 * 1024 - 64;   // 64 bytes for the static nlist
+    // d = 128: 8 waves (2 per SIMD, 192 VGPRs) of one row tile, 16 queries at
+    // G = 7, and 4 slots of 32 KB.  8192 tokens, 28 / 4 heads: 1.06 ms against
+    // 4.48 in bwd_dq_mfma (2048 tokens 0.12 against 0.53).  Two tiles per wave
+    // and 12 waves of one spill (77 and 35 VGPRs)
+    if constexpr (D == 128) {
+        if (dq_lds<128, 8, 1, 4>(n, G, k) <= LDS_MAX)
+            return launch_dq_t<128, 8, 1, 4, 2>(q, qgain, kgain, eps, kc, kr, v, cosT, sinT, idx, cnt, out, dout, B, n,
+                                                Hq, Hkv, S, W, k, scale, qc_ws, qr_ws, lse_ws, dd_ws, dq, dq_gain, s);
+        return HBA_ERR_UNSUPPORTED;
+    }
     // d = 64: 16 waves (4 per SIMD, within 128 VGPRs) of one row tile, 32
     // queries at G = 7; an 8-slot ring (4 blocks per phase) when the selection
     // lists fit beside it, else 4 slots.  Measured at 32K, this kernel alone:
@@ -1900,6 +1915,11 @@ int launch_attn_bf16_dq(const void *q, const float *qgain, const float *kgain, f
     return HBA_ERR_UNSUPPORTED;
 }
 template int launch_attn_bf16_dq<64>(const void *, const float *, const float *, float, const void *, const void *,
+                                     const void *, const float *, const float *,
+                                     const int32_t *, const int32_t *, const void *, const void *, int64_t, int64_t,
+                                     int64_t, int64_t, int64_t, int64_t, int64_t, float, void *, void *, float *,
+                                     float *, void *, float *, hipStream_t);
+template int launch_attn_bf16_dq<128>(const void *, const float *, const float *, float, const void *, const void *,
                                      const void *, const float *, const float *,
                                      const int32_t *, const int32_t *, const void *, const void *, int64_t, int64_t,
                                      int64_t, int64_t, int64_t, int64_t, int64_t, float, void *, void *, float *,

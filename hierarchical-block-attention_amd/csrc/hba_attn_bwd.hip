@@ -1034,11 +1034,10 @@ extern "C" int hba_attn_bwd(int dtype, const void *q, const void *k, const void 
 #define HBA_BWD(D)                                                                                              \
     do {                                                                                                        \
         int dqs = HBA_ERR_UNSUPPORTED;                                                                          \
-        if constexpr (D == 64)                                                                                  \
-            if (bwd_dq_union_on())                                                                              \
-                dqs = launch_attn_bf16_dq<D>(q, q_gain, k_gain, eps, kc, kr, v, cos_tab, sin_tab,                \
-                                             idx, cnt, out, dout, B, n, Hq, Hkv, S, W, k_blocks, scale,          \
-                                             qcb_ws, qrb_ws, lse_ws, dd_ws, dq, dq_gain, s);                     \
+        if (bwd_dq_union_on())                                                                                  \
+            dqs = launch_attn_bf16_dq<D>(q, q_gain, k_gain, eps, kc, kr, v, cos_tab, sin_tab, idx, cnt, out,     \
+                                         dout, B, n, Hq, Hkv, S, W, k_blocks, scale, qcb_ws, qrb_ws, lse_ws,     \
+                                         dd_ws, dq, dq_gain, s);                                                 \
         if (dqs != HBA_OK && dqs != HBA_ERR_UNSUPPORTED) return dqs;                                            \
         const bool kt = dqs != HBA_OK;                                                                          \
         hipLaunchKernelGGL((bw::bwd_kt_kernel<D>), dim3((unsigned)g2), dim3(256), 0, s, (const bf16_t *)kc,      \
