@@ -120,9 +120,10 @@ constexpr int DKV_ROWS = 4096;
 constexpr int PB_WORDS = DKV_ROWS / 32;
 
 // transposed prepared keys for bwd_dq_mfma, kct / krt [B, Hkv, d, n] (kct null:
-// none): one workgroup per 64-key tile; it also clears the tile's rows of the dk / dv accumulator dkv_acc
-// [B, Hkv, n, 3, d] (bwd_dkv_mfma adds into it next) and the tile's routed-row
-// bits of every range (bwd_pick_bits sets them next)
+// none): one workgroup per 64-key tile; it also clears the tile's rows of the
+// dk / dv accumulator dkv_acc [B, Hkv, n, 3, d] (bwd_dkv_mfma adds into it
+// next) and the tile's routed-row bits of every range (bwd_pick_bits sets them
+// next)
 template <int D>
 __global__ __launch_bounds__(256) void bwd_kt_kernel(const bf16_t *__restrict__ kc, const bf16_t *__restrict__ kr,
                                                      bf16_t *__restrict__ kct, bf16_t *__restrict__ krt, int64_t n,
@@ -896,8 +897,8 @@ __global__ __launch_bounds__(256) void bwd_dkv_fin_kernel(
 
 using namespace hba;
 
-// The bf16 query gradient: the union kernel (launch_attn_bf16_dq: 64 queries
-// per workgroup sharing each staged block) where it takes the geometry, else
+// The bf16 query gradient: the union kernel (launch_attn_bf16_dq: the queries
+// of a workgroup share each staged block) where it takes the geometry, else
 // bwd_dq_mfma.  HBA_BWD_DQ_KERNEL=pair in the environment selects
 // bwd_dq_mfma (16/G queries per wave) everywhere.
 static bool bwd_dq_union_on() {
