@@ -211,3 +211,24 @@ def test_backward_rows_outside_the_union_are_not_read_into_it():
     got = _run_bwd(q, kb, v, gq, gk, idx, cnt, dout, S, W)[0]
     sel = ((j >= 70) & (j < 70 + W)) | (j == 201)
     assert got[0][:, sel].isnan().all() and got[0][:, ~sel].isfinite().all()
+
+
+def test_backward_takes_rows_off_16_byte_boundaries():
+    """Contiguous fp32 tensors that begin 4 bytes past a 16-byte boundary."""
+    n, Hq, Hkv, d, S, W, k = shape = (192, 7, 1, 64, 4, 64, 3)
+    q, kx, v, gq, gk, idx, cnt = _inputs(*shape)
+    idx = _unique(idx, n)
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(5))
+    dev = torch.device("cuda")
+    cos, sin = hba_amd.rope_tables(n, d, 10000.0, dev)
+    t = [x.to(dev) for x in (q, kx, v, gq, gk, idx, cnt, dout)]
+    kc, kr, vt = ops.prep_keys(t[1], t[2], t[4], 1e-6, cos, sin)
+    out = ops.attn_fwd(t[0], t[3], t[4], 1e-6, kc, kr, vt, cos, sin, t[5], t[6], S, W, 0.125)
+
+    def off(x):
+        y = torch.empty(x.numel() + 1, dtype=x.dtype, device=dev)[1:].view(x.shape)
+        return y.copy_(x)
+    run = lambda f: ops.attn_bwd(f(t[0]), f(t[1]), f(t[2]), f(kc), f(kr), t[3], t[4], 1e-6, f(cos), f(sin), t[5], t[6],
+                                 f(out), f(t[7]), S, W, 0.125)
+    for a, b in zip(run(lambda x: x), run(off)):
+        assert (a - b).norm() <= 1e-6 * a.norm()       # the atomic sums' order
