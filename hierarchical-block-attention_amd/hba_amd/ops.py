@@ -42,7 +42,9 @@ def _code(t):
 # (a decode step at batch 1: 21 us of kernels, 51 us of host before, 38 so), so the helpers
 # below avoid what costs microseconds: wrapper objects for pointers and
 # streams, a device switch to the current device, and copies, views or
-# detached aliases of tensors that only lend their pointer.
+# detached aliases of tensors that only lend their pointer.  A copy that is
+# made for a call is held by a name until the call returns: only its pointer
+# would let the allocator give its memory to the next copy.
 def _p(t):
     return None if t is None else t.data_ptr()
 
@@ -392,17 +394,15 @@ def attn_fwd(q: Tensor, q_gain: Optional[Tensor], k_gain: Optional[Tensor], eps:
     cos, sin = _tables(cos, sin, n, d, dev)
     qg = _f32c(q_gain, dev, Hq, "q_gain")
     kg = _f32c(k_gain, dev, Hkv, "k_gain")
-    idx = idx.contiguous()
-    cnt = cnt.contiguous()
+    kc, kr, vt, idx, cnt = (t.contiguous() for t in (kc, kr, vt, idx, cnt))
     out = torch.empty(B, n, Hq, d, dtype=q.dtype, device=dev)
     nbytes = ctypes.c_size_t(0)
     check(lib().hba_attn_fwd_workspace_bytes(_code(q), B, n, Hq, d, ctypes.byref(nbytes)),
           "hba_attn_fwd_workspace_bytes")
     ws = torch.empty(max(int(nbytes.value), 16), dtype=torch.uint8, device=dev)
     with _on(dev):
-        st = lib().hba_attn_fwd(_code(q), _p(q), strides3(q), _p(qg), _p(kg), eps, _p(kc.contiguous()),
-                                _p(kr.contiguous()), _p(vt.contiguous()), _p(cos), _p(sin), _p(idx),
-                                _p(cnt), B, n, Hq, Hkv, d, sinks, window, block, idx.shape[3], scale,
+        st = lib().hba_attn_fwd(_code(q), _p(q), strides3(q), _p(qg), _p(kg), eps, _p(kc), _p(kr), _p(vt),
+                                _p(cos), _p(sin), _p(idx), _p(cnt), B, n, Hq, Hkv, d, sinks, window, block, idx.shape[3], scale,
                                 _p(ws), int(nbytes.value), _p(out), strides3(out), _stream(dev))
     check(st, "hba_attn_fwd")
     return out
@@ -433,10 +433,11 @@ def attn_window_(q, q_gain, k_gain, eps, kr, vt, cos, sin, sinks, window, scale,
     cos, sin = _tables(cos, sin, n, d, dev)
     qg = _f32c(q_gain, dev, Hq, "q_gain")
     kg = _f32c(k_gain, dev, Hkv, "k_gain")
+    kr, vt = kr.contiguous(), vt.contiguous()
     with _on(dev):
-        st = lib().hba_attn_window_fwd(_p(q), strides3(q), _p(qg), _p(kg), eps, _p(kr.contiguous()),
-                                       _p(vt.contiguous()), _p(cos), _p(sin), B, n, Hq, Hkv, d, sinks, window,
-                                       BLOCK, scale, _p(ws), ws.numel(), _p(out), strides3(out), _stream(dev))
+        st = lib().hba_attn_window_fwd(_p(q), strides3(q), _p(qg), _p(kg), eps, _p(kr), _p(vt), _p(cos), _p(sin),
+                                       B, n, Hq, Hkv, d, sinks, window, BLOCK, scale, _p(ws), ws.numel(), _p(out),
+                                       strides3(out), _stream(dev))
     check(st, "hba_attn_window_fwd")
     return out
 
@@ -457,13 +458,11 @@ def attn_routed_(q, q_gain, k_gain, eps, kc, vt, idx, cnt, sinks, scale, out, ws
         raise TypeError("idx/cnt must be int32")
     qg = _f32c(q_gain, dev, Hq, "q_gain")
     kg = _f32c(k_gain, dev, Hkv, "k_gain")
-    idx = idx.contiguous()
-    cnt = cnt.contiguous()
+    kc, vt, idx, cnt = (t.contiguous() for t in (kc, vt, idx, cnt))
     with _on(dev):
-        st = lib().hba_attn_routed_fwd(_p(q), strides3(q), _p(qg), _p(kg), eps, _p(kc.contiguous()),
-                                       _p(vt.contiguous()), _p(idx), _p(cnt), B, n, Hq, Hkv, d, sinks, BLOCK,
-                                       idx.shape[3], scale, _p(ws), ws.numel(), _p(out), strides3(out),
-                                       _stream(dev))
+        st = lib().hba_attn_routed_fwd(_p(q), strides3(q), _p(qg), _p(kg), eps, _p(kc), _p(vt), _p(idx), _p(cnt),
+                                       B, n, Hq, Hkv, d, sinks, BLOCK, idx.shape[3], scale, _p(ws), ws.numel(),
+                                       _p(out), strides3(out), _stream(dev))
     check(st, "hba_attn_routed_fwd")
     return out
 
@@ -548,8 +547,9 @@ def kv_append(k_new: Tensor, v_new: Tensor, k_gain: Optional[Tensor], eps: float
     Bd, Hkv, d = k_new.shape
     kg = _f32c(k_gain, dev, Hkv, "k_gain")
     cos, sin = _tables(cos, sin, 1, d, dev)
+    k_new, v_new = k_new.contiguous(), v_new.contiguous()
     with _on(dev):
-        st = lib().hba_kv_append(_code(k_new), _p(k_new.contiguous()), _p(v_new.contiguous()), _p(kg), eps,
+        st = lib().hba_kv_append(_code(k_new), _p(k_new), _p(v_new), _p(kg), eps,
                                  _p(cos), _p(sin), cos.shape[0], _p(page_table), page_table.shape[1],
                                  _p(seq_lens), Bd, Hkv, d, BLOCK, _p(kc_pages), _p(kr_pages), _p(v_pages),
                                  _stream(dev))
@@ -578,8 +578,9 @@ def kv_append_advance(k_new: Tensor, v_new: Tensor, k_gain: Optional[Tensor], ep
             raise ValueError(f"{what} must be a contiguous {dt} tensor on {dev}")
     if seq_lens.numel() != Bd or scales.numel() != Bd:
         raise ValueError(f"seq_lens and scales must hold {Bd} entries")
+    k_new, v_new = k_new.contiguous(), v_new.contiguous()
     with _on(dev):
-        st = lib().hba_kv_append_advance(_code(k_new), _p(k_new.contiguous()), _p(v_new.contiguous()), _p(kg), eps,
+        st = lib().hba_kv_append_advance(_code(k_new), _p(k_new), _p(v_new), _p(kg), eps,
                                          _p(cos), _p(sin), cos.shape[0], _p(page_table), page_table.shape[1],
                                          _p(seq_lens), Bd, Hkv, d, BLOCK, _p(kc_pages), _p(kr_pages), _p(v_pages),
                                          _p(pr), _p(pj), m, _p(summ_pages), _p(scale_tab), scale_tab.numel(),
