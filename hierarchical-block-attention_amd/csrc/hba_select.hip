@@ -190,6 +190,30 @@ constexpr int flat_waves() {   // the lists fill 64 KB of LDS
     return KMAX <= 16 ? 8 : 4;
 }
 
+// Whether the split pays: one wave per 64 queries (score_select_kernel) leaves
+// the chip idle or keeps it busy with `waves` wavefronts, each scoring `ncand`
+// blocks of `m` slots; the split adds a list per wave and their ranking, about
+// what a few dozen slots cost.  Times in us, one wave per 64 queries against
+// the split, 8 KV heads of 2 query heads, d = 64, unless stated:
+//  * under a wave per SIMD (1024) what counts is the chain of one wave, its
+//    slots and its heads' set-up.  1 candidate of 4 slots, 32 waves: 8.8, 13.8;
+//    13 of 1, 128 waves: 15.5, 16.5; 13 of 4: 27.0, 17.9; 13 of 1 with 16 heads
+//    and lists of 32: 50.2, 40.5.
+//  * under two: 61 of 1 (7 heads) 83, 107; 29 of 4 (7 heads) 91, 83.
+//  * past that the slots have to outweigh the lists; their scores cost more at
+//    d = 128, and lists of 16 split over eight waves, those of 32 over four.
+//    4096 waves: 61 of 4 285, 324, lists of 32 477, 400; 61 of 8 500, 467; d =
+//    128: 29 of 4 497, 537, 61 of 4 843, 746.  With one slot a block's insertion
+//    outweighs its score: 61 of 1 125, 267, and 254 of 1 at 8192 waves 563, 1069.
+template <int D, int KMAX>
+static bool flat_split(int64_t waves, int64_t ncand, int64_t m, int64_t G) {
+    constexpr bool L32 = KMAX > 16;
+    const int64_t slots = ncand * m;
+    if (waves < 1024) return slots + (L32 ? 2 * G : G) >= 27 && (L32 || ncand >= flat_waves<KMAX>() / 2);
+    if (waves < 2048) return slots >= 96;
+    return m > 1 && slots * D * D >= (L32 ? 975000 : 1950000);
+}
+
 template <int D, int M, int KMAX>
 __global__ __launch_bounds__(64 * flat_waves<KMAX>()) void score_select_f32_kernel(
     const float *__restrict__ q, int64_t qsb, int64_t qsn, int64_t qsh, const float *__restrict__ qgain, float eps,
@@ -1807,15 +1831,17 @@ void launch_flat(const void *q, const int64_t *qs, const float *qgain, float eps
         }
     }
     // (64-entry lists and their ranks do not fit a lane's registers)
-    if constexpr (DT == 0 && KMAX <= 32)
-        hipLaunchKernelGGL((score_select_f32_kernel<D, M, KMAX>), grid, dim3(64 * flat_waves<KMAX>()), 0, s,
-                           (const float *)q, qs[0], qs[1], qs[2], qgain, eps, (const float *)S0, n, (int)Hq, (int)Hkv,
-                           n / 64, W, (int)k, scale, idx, val, cnt, scores);
-    else
-        hipLaunchKernelGGL((score_select_kernel<DT, D, M, KMAX>), grid, dim3(SEL_WG), 0, s,
-                           (const typename St<DT>::T *)q, qs[0], qs[1], qs[2], qgain, eps,
-                           (const typename St<DT>::T *)S0, n, (int)Hq, (int)Hkv, n / 64, W, (int)k,
-                           scale, idx, val, cnt, scores);
+    if constexpr (DT == 0 && KMAX <= 32) {
+        if (flat_split<D, KMAX>(B * Hkv * (n / 64), cand_bmax(n - 1, 64, W), M, Hq / Hkv)) {
+            hipLaunchKernelGGL((score_select_f32_kernel<D, M, KMAX>), grid, dim3(64 * flat_waves<KMAX>()), 0, s,
+                               (const float *)q, qs[0], qs[1], qs[2], qgain, eps, (const float *)S0, n, (int)Hq,
+                               (int)Hkv, n / 64, W, (int)k, scale, idx, val, cnt, scores);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((score_select_kernel<DT, D, M, KMAX>), grid, dim3(SEL_WG), 0, s,
+                       (const typename St<DT>::T *)q, qs[0], qs[1], qs[2], qgain, eps, (const typename St<DT>::T *)S0, n,
+                       (int)Hq, (int)Hkv, n / 64, W, (int)k, scale, idx, val, cnt, scores);
 }
 
 // Workspace of the grouped level 2 (hier_l2_kernel): the routing queries

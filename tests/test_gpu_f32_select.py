@@ -19,6 +19,10 @@ pytestmark = pytest.mark.gpu
     (40, 100, 4, 2, 64, 2, 17),       # lists of 32: four waves
     (70, 64, 3, 1, 128, 8, 32),
     (80, 64, 2, 2, 128, 4, 64),       # lists of 64: one wave per 64 queries
+    (6, 64, 2, 1, 64, 8, 4),          # four candidates for eight waves
+    (3, 64, 16, 1, 64, 1, 20),        # one candidate, sixteen heads: four waves
+    (64, 64, 16, 16, 64, 1, 9),       # the chip full: one wave per 64 queries, lists of 16
+    (64, 64, 16, 16, 64, 1, 20),      # and of 32
 ])
 def test_flat_fp32_selection_is_exact(nb, W, Hq, Hkv, d, m, k):
     n, dev = 64 * nb, torch.device("cuda")
