@@ -1216,9 +1216,12 @@ __global__ __launch_bounds__(RtCfg<D>::NTHR, RtCfg<D>::NTHR / 256) void attn_rou
 // the key-gradient kernels the QKNorm'd and rotated rows (bf16), the LSE
 // (natural log) and D.
 //
-// No VGPR may spill here: the compiler has placed the spill of a value that
-// lives past a divergent loop before the loop's exec restore, where it stores
-// nothing (the LSE rows of a build with 16 spilled VGPRs all went to head 0).
+// Register pressure is kept where no VGPR spills: the compiler has placed the
+// spill of a value that lives past a divergent loop before the loop's exec
+// restore, where it stores nothing (the LSE rows of a build with 16 spilled
+// VGPRs all went to head 0).  The build refuses any kernel whose code has a
+// vector instruction in that place (lost_spills of hba_amd/build.py); the
+// kernels that spill (the routed attention, the fp32 d = 128 ones) have none.
 template <int D, int WAVES>
 struct DqCfg {
     static constexpr int NKS = D / 32;
