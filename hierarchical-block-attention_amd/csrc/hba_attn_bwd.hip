@@ -907,9 +907,10 @@ static bool bwd_dq_union_on() {
 }
 
 // Workspace of hba_attn_bwd: the query rows in the storage type (QKNorm'd,
-// rotated), LSE and D per (head, row), an unused [B, Hkv, 2, 64, d] fp32 (the
-// sizes are part of the ABI); on the bf16 path also the transposed keys kct, krt
-// [B, Hkv, d, n] and the fp32 dk / dv accumulators [B, Hkv, n, 3, d].
+// rotated), LSE and D per (head, row), the sink keys' sums of the fp32 path
+// [B, Hkv, 2, 64, d] (unused on the bf16 path; the sizes are part of the ABI); on
+// the bf16 path also the transposed keys kct, krt [B, Hkv, d, n] and the fp32 dk /
+// dv accumulators [B, Hkv, n, 3, d].
 namespace {
 struct BwdWs {
     size_t qc, qr, lse, dd, sink, kct, krt, dkv, pbits, total;
@@ -947,6 +948,16 @@ extern "C" int hba_attn_bwd_workspace_bytes(int dtype, int64_t B, int64_t n, int
     if (dtype != HBA_DTYPE_F32 && dtype != HBA_DTYPE_BF16) return HBA_ERR_UNSUPPORTED;
     *bytes = bwd_ws_layout(dtype, B, n, Hq, Hkv, d).total;
     if (dtype == HBA_DTYPE_F32) *bytes = std::max(*bytes, gen_bwd_ws_bytes(B, n, Hkv, d));   // the generic path
+    return HBA_OK;
+}
+
+extern "C" int hba_attn_bwd_workspace_full_bytes(int dtype, int64_t B, int64_t n, int64_t Hq, int64_t Hkv, int64_t d,
+                                                 size_t *bytes) {
+    const int st = hba_attn_bwd_workspace_bytes(dtype, B, n, Hq, Hkv, d, bytes);
+    if (st) return st;
+    // (other geometry takes the generic path, which has one size)
+    if (dtype == HBA_DTYPE_F32 && (d == 64 || d == 128) && n % 64 == 0 && Hq / Hkv <= bw::BW_GMAX)
+        *bytes = std::max(*bytes, bwd_ws_layout(dtype, B, n, Hq, Hkv, d).total + attn_bwd_f32_part_bytes(B, n, Hkv, d));
     return HBA_OK;
 }
 
@@ -1012,7 +1023,8 @@ extern "C" int hba_attn_bwd(int dtype, const void *q, const void *k, const void 
         const auto bwd = d == 64 ? launch_attn_bwd_f32<64> : launch_attn_bwd_f32<128>;
         st = bwd((const float *)q, (const float *)k, (const float *)v, (const float *)kc, (const float *)kr, q_gain,
                  k_gain, eps, cos_tab, sin_tab, idx, cnt, (const float *)out, (const float *)dout, B, n, Hq, Hkv, S, W,
-                 k_blocks, scale, (float *)(wsb + L.qc), (float *)(wsb + L.qr), lse_ws, dd_ws, (float *)dq, (float *)dk,
+                 k_blocks, scale, (float *)(wsb + L.qc), (float *)(wsb + L.qr), lse_ws, dd_ws,
+                 (float *)(wsb + L.sink), (float *)(wsb + L.total), ws_bytes - L.total, (float *)dq, (float *)dk,
                  (float *)dv, dq_gain, dk_gain, s);
         if (st) return st;
         HBA_LAUNCH_CHECK();

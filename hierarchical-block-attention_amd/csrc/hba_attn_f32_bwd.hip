@@ -10,9 +10,16 @@
 //   bwd_dkv_f32: a wave takes 16 keys of a 64-key block and the (query, head)
 //                pairs of a range of query rows that attend them, 16 per
 //                tile: S = X . K^T, dP = dO . V^T, dV += P^T . dO,
-//                dK += dS^T . X.  The ranges' sums meet in dk and dv by fp32
-//                atomics.
-//   bwd_k_f32:   the QKNorm backward of the key rows, in place.
+//                dK += dS^T . X.
+//   bwd_k_f32:   the ranges' sums added to dk and dv, and the QKNorm backward
+//                of the key rows.
+// dk and dv are the same bits from run to run, and with any workspace: a
+// launch of bwd_dkv_f32 takes as many ranges as there are places for their sums
+// beyond the workspace that hba_attn_bwd asks for, bwd_k_f32 adds these in order,
+// and with fewer than two places each range is a launch that adds to dk and dv
+// itself.  Atomic sums, in another order each time, cost 1 % less at 2048 tokens,
+// 14 / 2 heads, head dim 64 (992 us per training step against 1002), up to 10 %
+// less (8192 tokens, 8 heads: 1412 us against 1552, four launches of 8 ranges).
 //
 // Matrix cores bound all three products at 64 FLOP per SIMD and cycle; every
 // operand comes from L1 / L2 in the layout it is used in (16 bytes per lane,
@@ -49,8 +56,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dq_f32_kernel(
     const float *__restrict__ sinT, const int32_t *__restrict__ idx, const int32_t *__restrict__ cnt,
     const float *__restrict__ out, const float *__restrict__ dout, int n, int Hq, int Hkv, int S, int W, int kk,
     float scale, int ntiles, int Cn, int xmap, float *__restrict__ qc_ws, float *__restrict__ qr_ws,
-    float *__restrict__ lse_ws, float *__restrict__ dd_ws, float *__restrict__ dq, float *__restrict__ dk,
-    float *__restrict__ dv, float *__restrict__ dq_gain) {
+    float *__restrict__ lse_ws, float *__restrict__ dd_ws, float *__restrict__ dq, float *__restrict__ dq_gain) {
     constexpr int KT = 16, NC = D / 16, NM = KT / 16;
     __shared__ float gsum[4][16];
     int combo, wt;
@@ -76,12 +82,6 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dq_f32_kernel(
         const float *cs = cosT + (int64_t)ic * D, *sn = sinT + (int64_t)ic * D;
         Units<KT> u;
         u.init(idx, cnt, bh * n + i0, n, S, W, kk, qpt, i0);
-        // bwd_dkv_f32 adds into the key rows of these positions next
-        for (int r = i0; r <= u.ilast; ++r)
-            for (int t = lane; t < D; t += 64) {
-                dk[((b * n + r) * Hkv + g) * D + t] = 0.0f;
-                dv[((b * n + r) * Hkv + g) * D + t] = 0.0f;
-            }
         f32x4 x[NC], dO[NC], O[NC], On[NC], kf[NM][NC], vf[NM][NC];
         float ms, r, dd = 0.0f;
         q_load<D>(q + row - 4 * lg, ok, qgain ? qgain + h : nullptr, eps, lg, x, ms, r);
@@ -283,33 +283,39 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dq_f32_kernel(
 }
 
 // Workgroup (b, g, range of R query rows, 64-key block); the block index nb
-// stands for the sink keys of block 0, which every row from j on attends.
+// stands for the sink keys of block 0, which every row from j on attends.  A
+// launch takes the nr ranges from split0 on.  Slot ((b, g), block, range) of
+// `part` is [4 waves][dk, dv][D / 16][64 lanes] f32x4 (lane (l16, lg), e: key 4
+// lg + e of the wave's 16, element 16 c + l16); `used` says per slot and wave
+// whether it was written.  DIRECT (nr = 1) adds the sums to dk and dv, the
+// sinks' to `part`, a slot per (b, g).
 // About 32 ranges per sequence balance the blocks' rows (a block that many
 // queries picked, a range that a window only touches): at 2048 tokens, 14 / 2
 // heads, ranges of 256 rows took 424 us, 128 303, 64 263; at 4096 256 853, 128
 // 790.  Past 64K tokens ranges stay at 2048 rows, so that the list fits LDS.
 constexpr int F32_RMIN = 64, F32_RMAX = 2048;
 
-template <int D>
+template <int D, bool DIRECT>
 __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dkv_f32_kernel(
     const float *__restrict__ kc, const float *__restrict__ kr, const float *__restrict__ v,
     const float *__restrict__ cosT, const float *__restrict__ sinT, const int32_t *__restrict__ idx,
     const int32_t *__restrict__ cnt, const float *__restrict__ dout, int n, int Hq, int Hkv, int S, int W, int kk,
-    float scale, int R, int nsplit, int nblk, const float *__restrict__ qc_ws, const float *__restrict__ qr_ws,
-    const float *__restrict__ lse_ws, const float *__restrict__ dd_ws, float *__restrict__ dk,
-    float *__restrict__ dv) {
+    float scale, int R, int split0, int nr, int nblk, const float *__restrict__ qc_ws,
+    const float *__restrict__ qr_ws, const float *__restrict__ lse_ws, const float *__restrict__ dd_ws,
+    float *__restrict__ part, int *__restrict__ used, float *__restrict__ dk, float *__restrict__ dv) {
     constexpr int NC = D / 16;
     __shared__ int rows[F32_RMAX];
     __shared__ int wcount[4];
     const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lg = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nb = n / 64, G = Hq / Hkv;
-    const int bx = (int)(blockIdx.x % nblk), split = (int)((blockIdx.x / nblk) % nsplit);
-    const int64_t bg = blockIdx.x / ((int64_t)nblk * nsplit), b = bg / Hkv;
+    const int bx = (int)(blockIdx.x % nblk), sp = (int)((blockIdx.x / nblk) % nr);
+    const int64_t bg = blockIdx.x / ((int64_t)nblk * nr), b = bg / Hkv;
+    const int64_t slot = (DIRECT ? bg : (bg * nblk + bx) * nr + sp) * 4 + w;
     const int g = (int)(bg % Hkv);
     const bool sinks = bx == nb;
     const int blk = sinks ? 0 : bx;
-    const int r0 = split * R, r1 = min(n, r0 + R);
+    const int r0 = (split0 + sp) * R, r1 = min(n, r0 + R);
 
     // the range's rows that picked the block, ascending
     int nrt = 0;
@@ -335,11 +341,11 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dkv_f32_kernel(
         }
     }
     // from here on each wave is alone
-    if (sinks && 16 * w >= S) return;
     const int j0 = 64 * blk + 16 * w, j = j0 + l16;
     const int wa = max(j0, r0), wb = sinks ? -1 : min(min(n, j0 + 16 + W - 1), r1);   // window rows [wa, wb)
-    if (!sinks && wb <= wa && nrt == 0) return;
-    if (sinks && r1 <= j0) return;
+    const bool any = sinks ? (16 * w < S && r1 > j0) : (wb > wa || nrt > 0);
+    if (!DIRECT && lane == 0) used[slot] = any;
+    if (!any && (!DIRECT || split0 > 0)) return;
     const uint32_t magic = 0xffffffffu / (uint32_t)G + 1u;   // G > 1: u / G = umulhi(u, magic) for u < 2^16
     const int64_t qb = b * n * Hq * D;
     f32x4 kf[NC], vf[NC], gk[NC], gv[NC];
@@ -445,6 +451,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dkv_f32_kernel(
     for (int safe = 0;; safe = 1) {
 #pragma unroll
         for (int c = 0; c < NC; ++c) gk[c] = gv[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (DIRECT && !any) break;
         if (sinks) {
             load_k(kc);
             const int ra = max(r0, j0);
@@ -477,84 +484,213 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dkv_f32_kernel(
         for (int c = 0; c < NC; ++c) fin = fin && finite4(gk[c]) && finite4(gv[c]);
         if (safe || __all(fin)) break;
     }
+    const bool plus = DIRECT && split0 > 0;
+    if (!DIRECT || sinks) {
+        float *pp = part + slot * (2 * 16 * D) + 4 * lane;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            f32x4 *pk = reinterpret_cast<f32x4 *>(pp + 256 * c), *pv = reinterpret_cast<f32x4 *>(pp + 256 * (NC + c));
+            *pk = plus ? *pk + gk[c] : gk[c];
+            *pv = plus ? *pv + gv[c] : gv[c];
+        }
+        return;
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        if (sinks && j0 + 4 * lg + e >= S) continue;
         const int64_t o = ((b * n + j0 + 4 * lg + e) * Hkv + g) * D + l16;
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-            unsafeAtomicAdd(dk + o + 16 * c, gk[c][e]);
-            unsafeAtomicAdd(dv + o + 16 * c, gv[c][e]);
+            dk[o + 16 * c] = plus ? dk[o + 16 * c] + gk[c][e] : gk[c][e];
+            dv[o + 16 * c] = plus ? dv[o + 16 * c] + gv[c][e] : gv[c][e];
         }
     }
 }
 
-// The QKNorm backward of key rows, in place on dk: a workgroup takes a 64-key
-// block of one (b, g), lanes over d; one gain atomic per workgroup.
+// dk and dv of a 64-key block of one (b, g), a wave its 16 keys.  With `part`,
+// its nr ranges' sums are added to those of the earlier launches (in dk and dv,
+// the sinks' in `sink`; none if this is the first).  After the last launch of
+// ranges the sinks' sums are added to block 0 and the key rows taken through
+// the QKNorm backward, with one gain atomic per workgroup.
 template <int D>
-__global__ __launch_bounds__(256) void bwd_k_f32_kernel(const float *__restrict__ k, const float *__restrict__ kgain,
-                                                        float eps, int64_t n, int Hkv, float *__restrict__ dk,
-                                                        float *__restrict__ dk_gain) {
-    constexpr int E = D / 64;
+__global__ __launch_bounds__(256) void bwd_k_f32_kernel(const float *__restrict__ part, const int *__restrict__ used,
+                                                        float *__restrict__ sink, int nr, int nblk, int S, bool first,
+                                                        bool last, const float *__restrict__ k, const float *__restrict__ kgain,
+                                                        float eps, int n, int Hkv, float *__restrict__ dk,
+                                                        float *__restrict__ dv, float *__restrict__ dk_gain) {
+    constexpr int NC = D / 16, U = (D == 64) ? 4 : 2;
     __shared__ float gsum[4];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t bg = blockIdx.x / (n / 64), b = bg / Hkv;
+    const int lane = threadIdx.x & 63, l16 = lane & 15, lg = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nb = n / 64, blk = (int)(blockIdx.x % nb);
+    const int64_t bg = blockIdx.x / nb, b = bg / Hkv;
     const int g = (int)(bg % Hkv);
-    const float gn = kgain[g];
-    float gs = 0.0f;
-    for (int rr = 0; rr < 16; ++rr) {
-        const int64_t j = (blockIdx.x % (n / 64)) * 64 + 16 * w + rr;
-        const int64_t o = ((b * n + j) * Hkv + g) * D + lane;
-        float x[E], y[E], ss = 0.0f, yx = 0.0f;
+    const int64_t row = (b * n + 64 * (int64_t)blk + 16 * w + 4 * lg) * Hkv + g, rs = (int64_t)Hkv * D;
+    const int64_t o = row * D + l16;   // element 16 c of key e: o + e rs + 16 c
+    f32x4 gk[NC], gv[NC];
+    auto add = [&](int bx) {
+        const int64_t s0 = (bg * nblk + bx) * nr;
+        for (int c0 = 0; c0 < nr; c0 += 64) {
+            const bool u = c0 + lane < nr && used[(s0 + c0 + lane) * 4 + w] != 0;
+            for (uint64_t m = __ballot(u); m;) {   // U slots' loads in flight
+                f32x4 x[U][2 * NC];
+                bool has[U];
+                int i = 0;
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-            x[e] = k[o + 64 * e];
-            y[e] = dk[o + 64 * e];
-            ss = fmaf(x[e], x[e], ss);
-            yx = fmaf(y[e], x[e], yx);
+                for (int t = 0; t < U; ++t) {
+                    has[t] = m != 0;
+                    i = m ? __builtin_ctzll(m) : i;   // none left: the last one again, unused
+                    m &= m - 1;
+                    const float *pp = part + ((s0 + c0 + i) * 4 + w) * (2 * 16 * D) + 4 * lane;
+#pragma unroll
+                    for (int c = 0; c < 2 * NC; ++c) x[t][c] = ld4(pp + 256 * c);
+                }
+#pragma unroll
+                for (int t = 0; t < U; ++t)
+                    if (has[t]) {
+#pragma unroll
+                        for (int c = 0; c < NC; ++c) {
+                            gk[c] += x[t][c];
+                            gv[c] += x[t][NC + c];
+                        }
+                    }
+            }
         }
-        const float ms = wave_sum(ss) / (float)D;
-        yx = wave_sum(yx);
-        const float r = sqrtf(fmaxf(ms, eps));
-        const float corr = (ms >= eps) ? gn * yx / ((float)D * r * r * r) : 0.0f;
+    };
+    f32x4 *sp = reinterpret_cast<f32x4 *>(sink + (bg * 4 + w) * (2 * 16 * D)) + lane;
+    const bool sinks = blk == 0 && S > 16 * w;
+    if (part && sinks) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) dk[o + 64 * e] = (gn / r) * y[e] - x[e] * corr;
-        gs += yx / r;
+        for (int c = 0; c < NC; ++c) {
+            gk[c] = first ? f32x4{0.f, 0.f, 0.f, 0.f} : sp[64 * c];
+            gv[c] = first ? f32x4{0.f, 0.f, 0.f, 0.f} : sp[64 * (NC + c)];
+        }
+        add(nb);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            sp[64 * c] = gk[c];
+            sp[64 * (NC + c)] = gv[c];
+        }
     }
-    if (dk_gain) {
-        if (lane == 0) gsum[w] = gs;
-        __syncthreads();
-        if (threadIdx.x == 0) unsafeAtomicAdd(&dk_gain[g], (gsum[0] + gsum[1]) + (gsum[2] + gsum[3]));
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            gk[c][e] = first ? 0.0f : dk[o + e * rs + 16 * c];
+            gv[c][e] = first ? 0.0f : dv[o + e * rs + 16 * c];
+        }
+    if (part) add(blk);
+    if (last && sinks) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            gk[c] += sp[64 * c];
+            gv[c] += sp[64 * (NC + c)];
+        }
     }
+    if (last && kgain) {
+        const float gn = kgain[g];
+        float gs = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float x[NC], ss = 0.0f, yx = 0.0f;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                x[c] = k[o + e * rs + 16 * c];
+                ss = fmaf(x[c], x[c], ss);
+                yx = fmaf(gk[c][e], x[c], yx);
+            }
+#pragma unroll
+            for (int d = 1; d < 16; d *= 2) {   // over the key's 16 lanes
+                ss += __shfl_xor(ss, d, 64);
+                yx += __shfl_xor(yx, d, 64);
+            }
+            const float ms = ss / (float)D;
+            const float r = sqrtf(fmaxf(ms, eps));
+            const float corr = (ms >= eps) ? gn * yx / ((float)D * r * r * r) : 0.0f;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) gk[c][e] = (gn / r) * gk[c][e] - x[c] * corr;
+            gs += yx / r;
+        }
+        if (dk_gain) {
+            gs = col_sum(gs);
+            if (lane == 0) gsum[w] = gs;
+            __syncthreads();
+            if (threadIdx.x == 0) unsafeAtomicAdd(&dk_gain[g], (gsum[0] + gsum[1]) + (gsum[2] + gsum[3]));
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            dk[o + e * rs + 16 * c] = gk[c][e];
+            dv[o + e * rs + 16 * c] = gv[c][e];
+        }
+}
+
+// Ranges of query rows (R rows each, nsplit in all) and how many of them a
+// launch of bwd_dkv_f32 takes if the workspace has a place for each: enough for
+// F32_WGS workgroups (16 rounds of the 512 that run at once).  The places are
+// about F32_WGS times 32 KB at d = 64 then, however long the sequences are.  A
+// range of as many blocks or more fills the chip by itself and takes none.
+constexpr int64_t F32_WGS = 8192;
+struct Plan {
+    int64_t R, nsplit, nr;
+};
+static Plan bwd_plan(int64_t Cn, int64_t n) {
+    Plan p;
+    p.R = F32_RMIN;
+    while (n / p.R > 32 && p.R < F32_RMAX) p.R *= 2;
+    p.nsplit = (n + p.R - 1) / p.R;
+    const int64_t per = Cn * (n / 64 + 1);
+    p.nr = std::min(p.nsplit, (F32_WGS + per - 1) / per);
+    return p;
+}
+// one range's places: sums and flags
+static size_t range_bytes(int64_t Cn, int64_t n, int64_t d) {
+    return (size_t)(4 * Cn * (n / 64 + 1)) * (size_t)(2 * 16 * d + 1) * 4;
 }
 
 }  // namespace af
+
+size_t attn_bwd_f32_part_bytes(int64_t B, int64_t n, int64_t Hkv, int64_t d) {
+    const int64_t nr = af::bwd_plan(B * Hkv, n).nr;
+    return nr < 2 ? 0 : (size_t)nr * af::range_bytes(B * Hkv, n, d);
+}
 
 template <int D>
 int launch_attn_bwd_f32(const float *q, const float *k, const float *v, const float *kc, const float *kr,
                         const float *qgain, const float *kgain, float eps, const float *cosT, const float *sinT,
                         const int32_t *idx, const int32_t *cnt, const float *out, const float *dout, int64_t B,
                         int64_t n, int64_t Hq, int64_t Hkv, int64_t S, int64_t W, int64_t k_blocks, float scale,
-                        float *qc_ws, float *qr_ws, float *lse_ws, float *dd_ws, float *dq, float *dk, float *dv,
-                        float *dq_gain, float *dk_gain, hipStream_t s) {
-    const int64_t qpt = 16 / (Hq / Hkv), ntiles = ((n + qpt - 1) / qpt + 3) / 4, Cn = B * Hkv;
+                        float *qc_ws, float *qr_ws, float *lse_ws, float *dd_ws, float *sink, float *part,
+                        size_t part_bytes, float *dq, float *dk, float *dv, float *dq_gain, float *dk_gain,
+                        hipStream_t s) {
+    const int64_t qpt = 16 / (Hq / Hkv), ntiles = ((n + qpt - 1) / qpt + 3) / 4, Cn = B * Hkv, nb = n / 64;
     int64_t grid;
     const int xmap = xcd_pick(Cn, ntiles, grid);
-    int64_t R = af::F32_RMIN;
-    while (n / R > 32 && R < af::F32_RMAX) R *= 2;
-    const int64_t nsplit = (n + R - 1) / R, nblk = n / 64 + (S > 0), grid2 = Cn * nsplit * nblk;
-    if (grid > 0x7fffffffLL || grid2 > 0x7fffffffLL || n > 0x3fffffffLL || n * Hq > 0x7fffffffLL)
+    const af::Plan p = af::bwd_plan(Cn, n);
+    const int64_t places = std::min<int64_t>(p.nr, (int64_t)(part_bytes / af::range_bytes(Cn, n, D)));
+    const int64_t per = places < 2 ? 1 : places;   // ranges per launch
+    const int64_t nblk = nb + (S > 0);
+    if (grid > 0x7fffffffLL || Cn * nblk * per > 0x7fffffffLL || n > 0x3fffffffLL || n * Hq > 0x7fffffffLL)
         return HBA_ERR_UNSUPPORTED;
+    if (places < 2) part = nullptr;
+    int *used = part ? reinterpret_cast<int *>(part + 4 * Cn * nblk * per * (2 * 16 * D)) : nullptr;
     const int Wc = (int)std::min<int64_t>(W, n);   // past n a longer window changes nothing
     hipLaunchKernelGGL(af::bwd_dq_f32_kernel<D>, dim3((unsigned)grid), dim3(256), 0, s, q, kc, kr, v, qgain, eps, cosT,
                        sinT, idx, cnt, out, dout, (int)n, (int)Hq, (int)Hkv, (int)S, Wc, (int)k_blocks, scale,
-                       (int)ntiles, (int)Cn, xmap, qc_ws, qr_ws, lse_ws, dd_ws, dq, dk, dv, dq_gain);
-    hipLaunchKernelGGL(af::bwd_dkv_f32_kernel<D>, dim3((unsigned)grid2), dim3(256), 0, s, kc, kr, v, cosT, sinT, idx,
-                       cnt, dout, (int)n, (int)Hq, (int)Hkv, (int)S, Wc, (int)k_blocks, scale, (int)R, (int)nsplit,
-                       (int)nblk, qc_ws, qr_ws, lse_ws, dd_ws, dk, dv);
-    if (kgain)
-        hipLaunchKernelGGL(af::bwd_k_f32_kernel<D>, dim3((unsigned)(Cn * (n / 64))), dim3(256), 0, s, k, kgain, eps, n,
-                           (int)Hkv, dk, dk_gain);
+                       (int)ntiles, (int)Cn, xmap, qc_ws, qr_ws, lse_ws, dd_ws, dq, dq_gain);
+    const auto dkv = part ? af::bwd_dkv_f32_kernel<D, false> : af::bwd_dkv_f32_kernel<D, true>;
+    for (int64_t r0 = 0; r0 < p.nsplit; r0 += per) {
+        const int64_t nr = std::min(per, p.nsplit - r0);
+        const bool last = r0 + nr == p.nsplit;
+        hipLaunchKernelGGL(dkv, dim3((unsigned)(Cn * nblk * nr)), dim3(256), 0, s, kc, kr, v, cosT, sinT, idx, cnt,
+                           dout, (int)n, (int)Hq, (int)Hkv, (int)S, Wc, (int)k_blocks, scale, (int)p.R, (int)r0,
+                           (int)nr, (int)nblk, qc_ws, qr_ws, lse_ws, dd_ws, part ? part : sink, used, dk, dv);
+        if (part || (last && (kgain || S > 0)))
+            hipLaunchKernelGGL(af::bwd_k_f32_kernel<D>, dim3((unsigned)(Cn * nb)), dim3(256), 0, s, part, used, sink,
+                               (int)nr, (int)nblk, (int)S, part && r0 == 0, last, k, kgain, eps, (int)n, (int)Hkv, dk,
+                               dv, dk_gain);
+    }
     return HBA_OK;
 }
 #define HBA_INST(D)                                                                                                \
@@ -562,8 +698,8 @@ int launch_attn_bwd_f32(const float *q, const float *k, const float *v, const fl
                                         const float *, const float *, float, const float *, const float *,         \
                                         const int32_t *, const int32_t *, const float *, const float *, int64_t,   \
                                         int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, float, float *,      \
-                                        float *, float *, float *, float *, float *, float *, float *, float *,    \
-                                        hipStream_t);
+                                        float *, float *, float *, float *, float *, size_t, float *, float *,     \
+                                        float *, float *, float *, hipStream_t);
 HBA_INST(64)
 HBA_INST(128)
 #undef HBA_INST

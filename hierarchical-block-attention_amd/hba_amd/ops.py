@@ -519,9 +519,14 @@ def attn_bwd(q: Tensor, k: Tensor, v: Tensor, kc: Tensor, kr: Tensor, q_gain: Op
     dqg = torch.zeros(Hq, dtype=torch.float32, device=dev)
     dkg = torch.zeros(Hkv, dtype=torch.float32, device=dev)
     nbytes = ctypes.c_size_t(0)
-    check(lib().hba_attn_bwd_workspace_bytes(_code(q), B, n, Hq, Hkv, d, ctypes.byref(nbytes)),
-          "hba_attn_bwd_workspace_bytes")
-    ws = torch.empty(max(int(nbytes.value), 16), dtype=torch.uint8, device=dev)
+    check(lib().hba_attn_bwd_workspace_full_bytes(_code(q), B, n, Hq, Hkv, d, ctypes.byref(nbytes)),
+          "hba_attn_bwd_workspace_full_bytes")
+    try:
+        ws = torch.empty(max(int(nbytes.value), 16), dtype=torch.uint8, device=dev)
+    except torch.OutOfMemoryError:   # what it needs; the same bits in more launches
+        check(lib().hba_attn_bwd_workspace_bytes(_code(q), B, n, Hq, Hkv, d, ctypes.byref(nbytes)),
+              "hba_attn_bwd_workspace_bytes")
+        ws = torch.empty(max(int(nbytes.value), 16), dtype=torch.uint8, device=dev)
     with _on(dev):
         st = lib().hba_attn_bwd(_code(q), _p(q), _p(k), _p(v), _p(kc), _p(kr), _p(qg), _p(kg), eps, _p(cos),
                                 _p(sin), _p(idx), _p(cnt), _p(out), _p(dout), B, n, Hq, Hkv, d, sinks, window,

@@ -442,16 +442,18 @@ int hba_decode_fwd_noalloc(int dtype, const void *q, const float *q_gain, float 
  * (contiguous, storage dtype) and ADDS the QKNorm gain gradients into
  * dq_gain fp32 [Hq] and dk_gain fp32 [Hkv] (q_gain == NULL: no QKNorm, the
  * gain outputs are ignored).  scale is the union scale of the forward.
- * fp32 storage: fp32 VALU arithmetic.  bf16 storage: bf16 MFMA products
- * with fp32 accumulation; the probabilities and dS enter the dk/dv/dq
- * products rounded to bf16, and dk/dv are summed with fp32 atomics, so the
- * bf16 result is not bit-reproducible from run to run.  bf16: 64-key
- * blocks, d = 64 / 128, S <= 64, k <= 64, G = Hq/Hkv <= 16.  fp32 takes every
- * geometry the fp32 forward takes (any block size Bk dividing n up to 256,
- * even d <= 256, any S, k and G): off the tuned one, one thread per (query,
- * head) recomputes the union softmax and the key sides are summed with fp32
- * atomics (not bit-reproducible either); its workspace is three fp32
- * [B, Hkv, n, d] accumulators, included in hba_attn_bwd_workspace_bytes.
+ * fp32 storage: fp32 arithmetic, on the fp32 matrix cores at 64-key blocks,
+ * d = 64 / 128, S <= 64, k <= 64 and G = Hq/Hkv <= 16 (the tuned geometry); dq,
+ * dk and dv are the same bits from run to run there.  bf16 storage, on the
+ * same geometry only: bf16 MFMA products with fp32 accumulation; the
+ * probabilities and dS enter the dk/dv/dq products rounded to bf16, and dk/dv
+ * are summed with fp32 atomics, so they are not bit-reproducible.  fp32 takes
+ * every geometry the fp32 forward takes (any block size Bk dividing n up to
+ * 256, even d <= 256, any S, k and G): off the tuned one, one thread per
+ * (query, head) recomputes the union softmax and the key sides are summed with
+ * fp32 atomics (not bit-reproducible either); its workspace is three fp32
+ * [B, Hkv, n, d] accumulators, included in hba_attn_bwd_workspace_bytes.  The
+ * gain gradients are atomic sums everywhere.
  */
 int hba_attn_bwd(int dtype, const void *q, const void *k, const void *v,
                  const void *kc, const void *kr,
@@ -466,12 +468,22 @@ int hba_attn_bwd(int dtype, const void *q, const void *k, const void *v,
 
 /* Scratch bytes hba_attn_bwd needs for this dtype and Hkv: the QKNorm'd and
  * rotated query rows (2*B*n*Hq*d in the storage type), the per-row LSE and
- * <dout, out> (2*B*Hq*n fp32), an unused 2*B*Hkv*64*d fp32; on the bf16 path also the transposed prepared keys (2*B*Hkv*n*d
- * bf16), the dk/dv accumulators (3*B*Hkv*n*d fp32) and the routed-row bits
+ * <dout, out> (2*B*Hq*n fp32), the sink keys' sums of the fp32 path
+ * (2*B*Hkv*64*d fp32, in both); on the bf16 path also the transposed prepared
+ * keys (2*B*Hkv*n*d bf16), the dk/dv accumulators (3*B*Hkv*n*d fp32) and the routed-row bits
  * (B*Hkv*ceil(n/4096)*(n/64)*512 bytes: one bit per query row of each
  * 4096-row range and key block); each part rounded up to 256 bytes. */
 int hba_attn_bwd_workspace_bytes(int dtype, int64_t B, int64_t n, int64_t Hq, int64_t Hkv,
                                  int64_t d, size_t *bytes);
+
+/* hba_attn_bwd_workspace_bytes and what fp32 uses beyond it on the tuned
+ * geometry, for sums of dk and dv over ranges of query rows: places of
+ * B*Hkv*(n/64+1)*4 * (128*d + 4) bytes per range, for as many of the ceil(n/R)
+ * ranges (R rows: 64, doubled while n/R > 32, at most 2048) as make 8192 blocks.
+ * With fewer bytes the ranges run in more launches, down to one after another
+ * without a place; the results are the same bits. */
+int hba_attn_bwd_workspace_full_bytes(int dtype, int64_t B, int64_t n, int64_t Hq, int64_t Hkv,
+                                      int64_t d, size_t *bytes);
 
 /* An upper bound of hba_attn_bwd_workspace_bytes over both dtypes and every
  * Hkv <= Hq (for callers that size one workspace for any call). */

@@ -3,13 +3,14 @@ that fill, split and overflow a 16-column tile, pick lists of one and of
 several 64-pick chunks, repeated and invalid picks, sinks past the first
 block, windows of one key and of the whole sequence, and keys that are not
 finite outside a query's union."""
+import ctypes
 import math
 
 import pytest
 import torch
 
 import hba_amd
-from hba_amd import ops
+from hba_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -164,8 +165,9 @@ def _run_bwd(q, kx, v, gq, gk, idx, cnt, dout, S, W):
 
 #           n    Hq Hkv  d   S   W   k
 BWD_SHAPES = [s for s in SHAPES if s[4] <= 64 and s[6] <= 64 and s[1] // s[2] <= 16] + [
-    (832, 3, 1, 64, 17, 300, 4),       # 5 queries per tile, two sink waves, ranges of 256 rows, the last one ragged
-    (4608, 2, 2, 64, 4, 70, 3),        # one head per KV head, ranges of 512 rows
+    (832, 3, 1, 64, 17, 300, 4),       # 5 queries per tile, two sink waves, 13 ranges of 64 rows
+    (2112, 2, 1, 64, 4, 130, 3),       # 17 ranges of 128 rows, the last one ragged
+    (4608, 2, 2, 64, 4, 70, 3),        # one head per KV head, 18 ranges of 256 rows
 ]
 
 
@@ -232,3 +234,60 @@ def test_backward_takes_rows_off_16_byte_boundaries():
                                  f(out), f(t[7]), S, W, 0.125)
     for a, b in zip(run(lambda x: x), run(off)):
         assert (a - b).norm() <= 1e-6 * a.norm()       # the atomic sums' order
+
+
+def _bwd_args(shape, dev):
+    n, Hq, Hkv, d, S, W, k = shape
+    q, kx, v, gq, gk, idx, cnt = (x[:1] if x.dim() > 1 else x for x in _inputs(*shape))
+    idx = _unique(idx, n)
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(5))
+    cos, sin = hba_amd.rope_tables(n, d, 10000.0, dev)
+    t = [x.to(dev) for x in (q, kx, v, gq, gk, idx, cnt, dout)]
+    kc, kr, vt = ops.prep_keys(t[1], t[2], t[4], 1e-6, cos, sin)
+    out = ops.attn_fwd(t[0], t[3], t[4], 1e-6, kc, kr, vt, cos, sin, t[5], t[6], S, W, 0.125)
+    return t, kc, kr, cos, sin, out
+
+
+def test_backward_of_long_ranges_against_the_generic_kernels():
+    """17 ranges of 512 rows: two passes over the picks of each.  More than 64
+    picks per row, here unused ones, take the generic kernels."""
+    n, Hq, Hkv, d, S, W, k = shape = (8448, 2, 1, 64, 17, 300, 3)
+    t, kc, kr, cos, sin, out = _bwd_args(shape, torch.device("cuda"))
+    run = lambda idx: ops.attn_bwd(t[0], t[1], t[2], kc, kr, t[3], t[4], 1e-6, cos, sin, idx, t[6].clamp(max=k), out,
+                                   t[7], S, W, 0.125)
+    gen = run(torch.nn.functional.pad(t[5], (0, 65 - k), value=-1))
+    for name, a, b in zip(("dq", "dk", "dv"), run(t[5]), gen):
+        assert (a - b).norm() <= 1e-5 * b.norm(), name      # the bound of the 64-bit test, for either side
+
+
+#                                    n     Hq Hkv d   S   W    k
+@pytest.mark.parametrize("shape", [(2112, 6, 2, 64, 20, 130, 3), (832, 2, 1, 128, 4, 1000, 5), (192, 7, 1, 64, 0, 64, 3)])
+def test_backward_is_the_same_bits_from_run_to_run_and_with_any_workspace(shape):
+    """dq, dk and dv of two runs, and of a workspace with places for no, for
+    three and for all ranges of query rows."""
+    n, Hq, Hkv, d, S, W, k = shape
+    dev = torch.device("cuda")
+    t, kc, kr, cos, sin, out = _bwd_args(shape, dev)
+    lib, ws = _lib.lib(), {}
+    for name in ("bytes", "full_bytes"):
+        b = ctypes.c_size_t(0)
+        assert getattr(lib, "hba_attn_bwd_workspace_" + name)(0, 1, n, Hq, Hkv, d, ctypes.byref(b)) == 0
+        ws[name] = b.value
+    place = Hkv * (n // 64 + 1) * 4 * (128 * d + 4)
+    assert ws["full_bytes"] - ws["bytes"] == -(-n // (128 if n > 2048 else 64)) * place
+
+    def run(nbytes):
+        g = [torch.full_like(x, math.nan) for x in (t[0], t[1], t[2])]
+        gg = [torch.zeros_like(x) for x in (t[3], t[4])]
+        w = torch.full((nbytes,), 255, dtype=torch.uint8, device=dev)
+        p = lambda x: x.data_ptr()
+        st = lib.hba_attn_bwd(0, p(t[0]), p(t[1]), p(t[2]), p(kc), p(kr), p(t[3]), p(t[4]), 1e-6, p(cos), p(sin),
+                              p(t[5]), p(t[6]), p(out), p(t[7]), 1, n, Hq, Hkv, d, S, W, 64, k, 0.125, p(w), nbytes,
+                              *(p(x) for x in g + gg), torch.cuda.current_stream().cuda_stream)
+        assert st == 0
+        return g
+    want = ops.attn_bwd(t[0], t[1], t[2], kc, kr, t[3], t[4], 1e-6, cos, sin, t[5], t[6], out, t[7], S, W, 0.125)[:3]
+    assert all(x.isfinite().all() for x in want)
+    for nbytes in (ws["full_bytes"], ws["full_bytes"], ws["bytes"] + 3 * place + 64, ws["bytes"]):
+        for name, a, b in zip(("dq", "dk", "dv"), run(nbytes), want):
+            assert torch.equal(a, b), (name, nbytes)
