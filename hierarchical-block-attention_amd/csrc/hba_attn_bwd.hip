@@ -1044,10 +1044,12 @@ extern "C" int hba_attn_bwd(int dtype, const void *q, const void *k, const void 
     const int64_t gpb = (B * Hkv * n * k_blocks + 255) / 256;     // bwd_pick_bits: a thread per pick
     if (gpb > 0x7fffffffLL) return HBA_ERR_UNSUPPORTED;
     if (g3 > 0x7fffffffLL) return HBA_ERR_UNSUPPORTED;
+    // the union kernel copies rows of kc, kr and v into LDS in 16-byte pieces
+    const bool dma_ok = abi::aligned16(kc) && abi::aligned16(kr) && abi::aligned16(v);
 #define HBA_BWD(D)                                                                                              \
     do {                                                                                                        \
         int dqs = HBA_ERR_UNSUPPORTED;                                                                          \
-        if (bwd_dq_union_on())                                                                                  \
+        if (bwd_dq_union_on() && dma_ok)                                                                        \
             dqs = launch_attn_bf16_dq<D>(q, q_gain, k_gain, eps, kc, kr, v, cos_tab, sin_tab, idx, cnt, out,     \
                                          dout, B, n, Hq, Hkv, S, W, k_blocks, scale, qcb_ws, qrb_ws, lse_ws,     \
                                          dd_ws, dq, dq_gain, s);                                                 \

@@ -265,7 +265,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dq_f32_kernel(
         }
         if (ok) {
 #pragma unroll
-            for (int c = 0; c < NC; ++c) *reinterpret_cast<f32x4 *>(dq + row + 16 * c) = y[c];
+            for (int c = 0; c < NC; ++c) *reinterpret_cast<f32x4_a4 *>(dq + row + 16 * c) = y[c];
         }
     }
     // the gain gradient: one atomic per head and workgroup (the adds of all

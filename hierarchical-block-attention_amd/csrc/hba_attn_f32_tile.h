@@ -11,7 +11,9 @@ namespace af {
 __device__ __forceinline__ f32x4 mma4(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ f32x4 ld4(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
+// the backward's callers may pass rows off 16-byte boundaries
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+__device__ __forceinline__ f32x4 ld4(const float *p) { return *reinterpret_cast<const f32x4_a4 *>(p); }
 __device__ __forceinline__ bool finite4(f32x4 v) {
     return fabsf(v[0]) < INFINITY && fabsf(v[1]) < INFINITY && fabsf(v[2]) < INFINITY && fabsf(v[3]) < INFINITY;
 }

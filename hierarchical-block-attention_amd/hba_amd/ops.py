@@ -91,6 +91,12 @@ def _f32c(t, dev, n=None, what="tensor"):
     return t
 
 
+def _c16(t):
+    """Contiguous and on a 16-byte boundary, as the kernels' wide loads take rows."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _rows(t, what):
     if t.dim() != 4 or t.stride(3) != 1:
         raise ValueError(f"{what}: expected a [B, n, H, d] view with a contiguous last dim")
@@ -512,7 +518,7 @@ def attn_bwd(q: Tensor, k: Tensor, v: Tensor, kc: Tensor, kr: Tensor, q_gain: Op
     kg = _f32c(k_gain, dev, Hkv, "k_gain")
     if (qg is None) != (kg is None):
         raise ValueError("q_gain and k_gain are both given (QKNorm) or both None")
-    q, k, v, kc, kr, out, dout = (t.contiguous() for t in (q, k, v, kc, kr, out, dout))
+    q, k, v, kc, kr, out, dout = (_c16(t) for t in (q, k, v, kc, kr, out, dout))
     idx = idx.contiguous()
     cnt = cnt.contiguous()
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)

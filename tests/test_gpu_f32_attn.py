@@ -234,13 +234,38 @@ def test_backward_takes_rows_off_16_byte_boundaries():
                                  f(out), f(t[7]), S, W, 0.125)
     for a, b in zip(run(lambda x: x), run(off)):
         assert (a - b).norm() <= 1e-6 * a.norm()       # the atomic sums' order
+    # the C entry, which takes them as they are
+    for a, b in zip(_c_bwd(t, kc, kr, cos, sin, out, shape), _c_bwd([off(x) if x.dtype == torch.float32 else x for x in t],
+                                                                    off(kc), off(kr), off(cos), off(sin), off(out), shape)):
+        assert torch.equal(a, b)
 
 
-def _bwd_args(shape, dev):
+def _c_bwd(t, kc, kr, cos, sin, out, shape, nbytes=None):
+    """dq, dk and dv of hba_attn_bwd itself; gradients in memory aligned like the inputs."""
+    n, Hq, Hkv, d, S, W, k = shape
+    lib, dev, dt = _lib.lib(), kc.device, 0 if kc.dtype == torch.float32 else 1
+    if nbytes is None:
+        b = ctypes.c_size_t(0)
+        assert lib.hba_attn_bwd_workspace_bytes(dt, t[0].shape[0], n, Hq, Hkv, d, ctypes.byref(b)) == 0
+        nbytes = b.value
+    g = [torch.full((x.numel() + 8,), math.nan, dtype=x.dtype, device=dev)
+         [x.data_ptr() % 16 // x.element_size():][:x.numel()].view(x.shape) for x in t[:3]]
+    gg = [torch.zeros_like(x) for x in (t[3], t[4])]
+    ws = torch.full((nbytes,), 255, dtype=torch.uint8, device=dev)
+    p = lambda x: x.data_ptr()
+    st = lib.hba_attn_bwd(dt, p(t[0]), p(t[1]), p(t[2]), p(kc), p(kr), p(t[3]), p(t[4]), 1e-6, p(cos), p(sin), p(t[5]),
+                          p(t[6]), p(out), p(t[7]), t[0].shape[0], n, Hq, Hkv, d, S, W, 64, k, 0.125, p(ws), nbytes,
+                          *(p(x) for x in g + gg), torch.cuda.current_stream().cuda_stream)
+    assert st == 0
+    return g
+
+
+def _bwd_args(shape, dev, dt=torch.float32):
     n, Hq, Hkv, d, S, W, k = shape
     q, kx, v, gq, gk, idx, cnt = (x[:1] if x.dim() > 1 else x for x in _inputs(*shape))
+    q, kx, v = (x.to(dt) for x in (q, kx, v))
     idx = _unique(idx, n)
-    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(5))
+    dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(5)).to(dt)
     cos, sin = hba_amd.rope_tables(n, d, 10000.0, dev)
     t = [x.to(dev) for x in (q, kx, v, gq, gk, idx, cnt, dout)]
     kc, kr, vt = ops.prep_keys(t[1], t[2], t[4], 1e-6, cos, sin)
@@ -276,18 +301,31 @@ def test_backward_is_the_same_bits_from_run_to_run_and_with_any_workspace(shape)
     place = Hkv * (n // 64 + 1) * 4 * (128 * d + 4)
     assert ws["full_bytes"] - ws["bytes"] == -(-n // (128 if n > 2048 else 64)) * place
 
-    def run(nbytes):
-        g = [torch.full_like(x, math.nan) for x in (t[0], t[1], t[2])]
-        gg = [torch.zeros_like(x) for x in (t[3], t[4])]
-        w = torch.full((nbytes,), 255, dtype=torch.uint8, device=dev)
-        p = lambda x: x.data_ptr()
-        st = lib.hba_attn_bwd(0, p(t[0]), p(t[1]), p(t[2]), p(kc), p(kr), p(t[3]), p(t[4]), 1e-6, p(cos), p(sin),
-                              p(t[5]), p(t[6]), p(out), p(t[7]), 1, n, Hq, Hkv, d, S, W, 64, k, 0.125, p(w), nbytes,
-                              *(p(x) for x in g + gg), torch.cuda.current_stream().cuda_stream)
-        assert st == 0
-        return g
     want = ops.attn_bwd(t[0], t[1], t[2], kc, kr, t[3], t[4], 1e-6, cos, sin, t[5], t[6], out, t[7], S, W, 0.125)[:3]
     assert all(x.isfinite().all() for x in want)
     for nbytes in (ws["full_bytes"], ws["full_bytes"], ws["bytes"] + 3 * place + 64, ws["bytes"]):
-        for name, a, b in zip(("dq", "dk", "dv"), run(nbytes), want):
+        for name, a, b in zip(("dq", "dk", "dv"), _c_bwd(t, kc, kr, cos, sin, out, shape, nbytes), want):
             assert torch.equal(a, b), (name, nbytes)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_bf16_backward_takes_rows_off_16_byte_boundaries(d, monkeypatch):
+    """Keys and values 8 bytes past a boundary: the C entry's query gradient by
+    the kernel without 16-byte copies into LDS, the op's by the one with them."""
+    n, Hq, Hkv, d, S, W, k = shape = (192, 7, 1, d, 4, 64, 3)
+    dev = torch.device("cuda")
+    t, kc, kr, cos, sin, out = _bwd_args(shape, dev, torch.bfloat16)
+
+    def off(x):
+        y = torch.empty(x.numel() + 4, dtype=x.dtype, device=dev)[4:].view(x.shape)
+        return y.copy_(x)
+    moved = [off(x) if x.dtype == torch.bfloat16 else x for x in t]
+    run = lambda t, kc, kr: ops.attn_bwd(t[0], t[1], t[2], kc, kr, t[3], t[4], 1e-6, cos, sin, t[5], t[6], out, t[7], S, W,
+                                         0.125)[0]
+    assert torch.equal(run(t, kc, kr), run(moved, off(kc), off(kr)))
+    got = _c_bwd(moved, off(kc), off(kr), cos, sin, out, shape)
+    monkeypatch.setenv("HBA_BWD_DQ_KERNEL", "pair")
+    pair = _c_bwd(t, kc, kr, cos, sin, out, shape)
+    assert torch.equal(got[0], pair[0])
+    for a, b in zip(got[1:], pair[1:]):      # fp32 sums in any order, stored in bf16
+        assert (a.float() - b.float()).norm() <= 1e-2 * b.float().norm()
