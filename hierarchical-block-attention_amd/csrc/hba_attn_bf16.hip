@@ -548,7 +548,9 @@ __device__ __forceinline__ void win_body(
 
 // Grid: Cn = B*Hkv*hsplit combos (the heads of a group split over hsplit
 // workgroups of gw heads when G > 8) times the query tiles.
-template <int D, int RT>
+// ORDER 0: the tiles in eighths per XCD, 1: deepest first, 2: the one that xmap
+// says (< 0: eighths).
+template <int D, int RT, int ORDER>
 __global__ __launch_bounds__(256, 3) void attn_win_kernel(
     const bf16_t *__restrict__ q, int64_t qsb, int64_t qsn, int64_t qsh, const float *__restrict__ qgain,
     const float *__restrict__ kgain, float eps, const bf16_t *__restrict__ kr, const bf16_t *__restrict__ vt,
@@ -557,7 +559,7 @@ __global__ __launch_bounds__(256, 3) void attn_win_kernel(
     bf16_t *__restrict__ out, int64_t osb, int64_t osn, int64_t osh, float *__restrict__ lse) {
     extern __shared__ __align__(16) char smem[];
     int hs, tile, combo;
-    if (xmap < 0) {
+    if (ORDER == 0 || (ORDER == 2 && xmap < 0)) {
         // Work unit u = ((combo * ntiles + tile) * hsplit + hs), hs fastest.
         // XCD x (workgroup i runs on XCD i % 8) takes the x-th contiguous
         // eighth of the units, so the heads and neighbouring tiles that read
@@ -1722,20 +1724,32 @@ static int launch_win(const void *q, const int64_t *qs, const float *qgain, cons
     // their position, and an eighth of the units per XCD gives some XCDs the
     // deepest tiles only: deepest first over all of them instead.  Dense
     // causal attention of 8128 tokens, 14 / 2 heads, head dim 64: 310 us in
-    // eighths, 183 deepest first (943 against 1313 for 8192 tokens, 28 / 4 heads, head dim 128).  Tiles of a shorter window cost alike,
-    // and stay next to the tiles that read the same keys.
+    // eighths, 183 deepest first (943 against 1313 for 8192 tokens, 28 / 4
+    // heads, head dim 128).  Between half and all of the sequence (8192 tokens):
+    // 14 / 2 heads, d = 64, W = 4160 290 and 179, 6144 416 and 227; 8 / 8 heads
+    // 165 and 161, 224 and 199; 32 / 8, d = 128 865 and 830, 1065 and 1012; at
+    // 1024 to 16384 tokens and 1 to 4 sequences of these none slower.  Tiles of a
+    // shorter window cost alike, and stay next to the tiles that read the same
+    // keys.
     int64_t grid = 8 * ((U + 7) / 8);
-    const int xmap = 2 * W > n ? xcd_pick(B * Hkv, ntiles * hsplit, grid) : -1;
+    const bool deep = W > n / 2;
+    const int xmap = deep ? xcd_pick(B * Hkv, ntiles * hsplit, grid) : -1;
     if (grid > 0x7fffffff) return HBA_ERR_UNSUPPORTED;
     const size_t lds = (size_t)C::NS * C::SLOT * 2;
-    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_win_kernel<D, RT>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    // d = 128 takes a kernel per order (one for both: 2 % more for W = n / 2, 857
+    // and 875 us at 8192 tokens, 32 / 8 heads), d = 64 one for both (a kernel per
+    // order: 4 % more for W = n, 68 and 70 us at 2048 tokens, 14 / 2 heads)
+    auto kern = &attn_win_kernel<D, RT, D == 128 ? 1 : 2>;
+    if constexpr (D == 128)
+        if (!deep) kern = &attn_win_kernel<D, RT, 0>;
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)lds) != hipSuccess)
         return HBA_ERR_LAUNCH;
     const int Wc = (int)((W < n + 1) ? W : n + 1);     // a window longer than the sequence is the sequence
-    hipLaunchKernelGGL((attn_win_kernel<D, RT>), dim3((unsigned)grid), dim3(nthr), lds, s, (const bf16_t *)q, qs[0],
-                       qs[1], qs[2], qgain, kgain, eps, (const bf16_t *)kr, (const bf16_t *)vt, cosT, sinT, (int)n,
-                       (int)Hq, (int)Hkv, (int)S, Wc, scale, gw, hsplit, wsplit, (int)ntiles, (int)Cn, xmap,
-                       (bf16_t *)out, os[0], os[1], os[2], lse);
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(nthr), lds, s, (const bf16_t *)q, qs[0], qs[1], qs[2], qgain,
+                       kgain, eps, (const bf16_t *)kr, (const bf16_t *)vt, cosT, sinT, (int)n, (int)Hq, (int)Hkv,
+                       (int)S, Wc, scale, gw, hsplit, wsplit, (int)ntiles, (int)Cn, xmap, (bf16_t *)out, os[0], os[1],
+                       os[2], lse);
     return HBA_OK;
 }
 
