@@ -1239,7 +1239,7 @@ struct DqCfg {
     static constexpr int PPW = (NPARTS + WAVES - 1) / WAVES;   // DMA parts per wave per block, at most
 };
 
-enum { DQ_ALL = 0, DQ_COL = 1, DQ_RANGE = 2 };
+enum { DQ_COL, DQ_RANGE };
 
 // The MFMA operand x * f, rounded to bf16 (v_cvt_pk_bf16_f32).
 __device__ __forceinline__ bf16x8 scale8(bf16x8 x, float f) {
@@ -1249,10 +1249,9 @@ __device__ __forceinline__ bf16x8 scale8(bf16x8 x, float f) {
     return pack8(y);
 }
 
-// One staged block (K tile Ks, V tile Vk, K^T tile KT) against one 16-row
-// tile.  MODE DQ_ALL: every key of every column; DQ_COL: every key of the
-// columns whose query picked the block (colok); DQ_RANGE: keys jlo..jhi
-// (from the block's first key) of each column.  acc accumulates
+// One staged block (K tile Ks, V tile Vk) against one 16-row tile.  MODE
+// DQ_COL: every key of the columns whose query picked the block (colok);
+// DQ_RANGE: keys jlo..jhi (from the block's first key) of each column.  acc accumulates
 // sum_j p~_j (dP_j - D) k_j with p~ = exp2 of the score less the shift;
 // lsum (per lane: the lane's keys only) sum_j p~_j.  The V fragments are read
 // after the scores' exponentials, so that the K and V fragments are not live
@@ -1796,7 +1795,11 @@ static int launch_routed_t(const void *q, const int64_t *qs, const float *qgain,
 // unit (each column sums its blocks in the same order either way).  14 / 2
 // heads, d = 64, two tiles against one: 1216 tokens (38 workgroups of two) 54.6
 // and 32.0 us, 4096 (128) 116 and 70, 6144 (192) 131 and 107, 8192 (256) 146
-// and 143, 16384 (512) 301 and 337.
+// and 143, 16384 (512) 301 and 337.  Other groups, d = 64, 512 tokens of window:
+// 16 / 16 heads, 8192 tokens (256) 323 and 242; 32 / 8, 4096 (256) 152 and 127;
+// 16 / 1, 8192 (256) 122 and 123; four sequences of 2048, 14 / 2 (256) 103 and
+// 82; with 100 sinks and 16 picks 4096 tokens, 14 / 2 (128) 159 and 89, 32 / 8
+// (256) 194 and 140.
 constexpr int64_t CUS = 256;
 template <int D, bool WIN>
 static int launch_routed(const void *q, const int64_t *qs, const float *qgain, const float *kgain, float eps,

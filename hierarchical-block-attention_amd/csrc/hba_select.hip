@@ -190,28 +190,37 @@ constexpr int flat_waves() {   // the lists fill 64 KB of LDS
     return KMAX <= 16 ? 8 : 4;
 }
 
-// Whether the split pays: one wave per 64 queries (score_select_kernel) leaves
-// the chip idle or keeps it busy with `waves` wavefronts, each scoring `ncand`
-// blocks of `m` slots; the split adds a list per wave and their ranking, about
-// what a few dozen slots cost.  Times in us, one wave per 64 queries against
-// the split, 8 KV heads of 2 query heads, d = 64, unless stated:
-//  * under a wave per SIMD (1024) what counts is the chain of one wave, its
-//    slots and its heads' set-up.  1 candidate of 4 slots, 32 waves: 8.8, 13.8;
-//    13 of 1, 128 waves: 15.5, 16.5; 13 of 4: 27.0, 17.9; 13 of 1 with 16 heads
-//    and lists of 32: 50.2, 40.5.
-//  * under two: 61 of 1 (7 heads) 83, 107; 29 of 4 (7 heads) 91, 83.
-//  * past that the slots have to outweigh the lists; their scores cost more at
-//    d = 128, and lists of 16 split over eight waves, those of 32 over four.
-//    4096 waves: 61 of 4 285, 324, lists of 32 477, 400; 61 of 8 500, 467; d =
-//    128: 29 of 4 497, 537, 61 of 4 843, 746.  With one slot a block's insertion
-//    outweighs its score: 61 of 1 125, 267, and 254 of 1 at 8192 waves 563, 1069.
+// Whether the split pays.  One wave per 64 queries (score_select_kernel) leaves
+// the chip idle or keeps it busy with `waves` wavefronts, each scoring up to
+// `ncand` blocks of `m` slots.  The split shares the slots and the heads' set-up
+// over its waves and adds a list per wave and their ranking, a few dozen slots'
+// time for lists of 16 over eight waves, a dozen for lists of 32 over four.
+// Times in us, one wave per 64 queries and the split, 8 KV heads of 2 query heads,
+// d = 64, lists of 16 unless stated:
+//  * no candidates: the split's workgroups leave before the queries' set-up.
+//  * up to two workgroups of the split per compute unit the chain of one wave is
+//    what counts.  1 candidate of 4 slots, 32 waves: 9.1, 14.0; 6 of 4, 72 waves
+//    16.9, 15.4; 13 of 1, 128 waves 15.5, 16.5, lists of 32 20.6, 19.7, those with
+//    7 heads (2 KV heads) 30.9, 26.8.  At d = 128 scores and set-up weigh more,
+//    until a second workgroup waits for the first (past 256): 1 query head per KV
+//    head, 13 of 1, 128 waves 20.3, 18.4; 512 waves 23.1, 35.3.
+//  * up to four: 6 of 4, 864 waves 23.8, 31.0; 14 of 8, 544 waves 48.1, 28.8;
+//    lists of 32, 5 of 1, 768 waves 24.2, 35.5; 5 of 8 50.9, 47.5.
+//  * past that the slots have to outweigh the lists, and with few slots per block
+//    its insertion outweighs its scores.  4096 waves: 61 of 1 125, 267; 61 of 4
+//    285, 324, lists of 32 477, 400; 61 of 8 500, 467; d = 128 29 of 4 497, 537,
+//    61 of 4 843, 746.
 template <int D, int KMAX>
 static bool flat_split(int64_t waves, int64_t ncand, int64_t m, int64_t G) {
     constexpr bool L32 = KMAX > 16;
     const int64_t slots = ncand * m;
-    if (waves < 1024) return slots + (L32 ? 2 * G : G) >= 27 && (L32 || ncand >= flat_waves<KMAX>() / 2);
-    if (waves < 2048) return slots >= 96;
-    return m > 1 && slots * D * D >= (L32 ? 975000 : 1950000);
+    if (ncand == 0) return true;
+    if (waves <= 512) {
+        if (L32) return 2 * slots + (D == 64 ? 3 * G : 0) >= 28;
+        return ncand >= 3 && (slots + G) * (waves <= 256 ? D : 64) >= 23 * 64;
+    }
+    if (waves <= 1152) return L32 ? slots * m >= 120 : slots >= 80;
+    return L32 ? slots * m * D * D >= 850 * 4096 : slots * m * D >= 1950 * 64;
 }
 
 template <int D, int M, int KMAX>

@@ -400,7 +400,8 @@ def attn_fwd(q: Tensor, q_gain: Optional[Tensor], k_gain: Optional[Tensor], eps:
     cos, sin = _tables(cos, sin, n, d, dev)
     qg = _f32c(q_gain, dev, Hq, "q_gain")
     kg = _f32c(k_gain, dev, Hkv, "k_gain")
-    kc, kr, vt, idx, cnt = (t.contiguous() for t in (kc, kr, vt, idx, cnt))
+    kc, kr, vt = kc.contiguous(), kr.contiguous(), vt.contiguous()
+    idx, cnt = idx.contiguous(), cnt.contiguous()
     out = torch.empty(B, n, Hq, d, dtype=q.dtype, device=dev)
     nbytes = ctypes.c_size_t(0)
     check(lib().hba_attn_fwd_workspace_bytes(_code(q), B, n, Hq, d, ctypes.byref(nbytes)),
@@ -464,7 +465,8 @@ def attn_routed_(q, q_gain, k_gain, eps, kc, vt, idx, cnt, sinks, scale, out, ws
         raise TypeError("idx/cnt must be int32")
     qg = _f32c(q_gain, dev, Hq, "q_gain")
     kg = _f32c(k_gain, dev, Hkv, "k_gain")
-    kc, vt, idx, cnt = (t.contiguous() for t in (kc, vt, idx, cnt))
+    kc, vt = kc.contiguous(), vt.contiguous()
+    idx, cnt = idx.contiguous(), cnt.contiguous()
     with _on(dev):
         st = lib().hba_attn_routed_fwd(_p(q), strides3(q), _p(qg), _p(kg), eps, _p(kc), _p(vt), _p(idx), _p(cnt),
                                        B, n, Hq, Hkv, d, sinks, BLOCK, idx.shape[3], scale, _p(ws), ws.numel(),
