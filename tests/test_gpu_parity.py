@@ -1058,7 +1058,7 @@ def test_backward_bf16_cases(dev, case):
 @pytest.mark.parametrize("n", [32768, 65536])
 def test_backward_dq_kernels_agree(dev, n):
     """The bf16 query gradient at the benchmarked 32K shape (14/2 heads, d =
-    64, W = 1024, k = 16, needles; a 6-slot ring) and at 64K (a 4-slot ring:
+    64, W = 1024, k = 16, needles; an 8-slot ring) and at 64K (a 4-slot ring:
     the selection lists take more LDS): the union kernel (64-key blocks
     staged once per 48 queries) against bwd_dq_mfma (HBA_BWD_DQ_KERNEL=pair),
     which the oracle tests pin at small n.  Both compute the same sums in a
