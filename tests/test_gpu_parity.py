@@ -1060,7 +1060,7 @@ def test_backward_dq_kernels_agree(dev, n):
     """The bf16 query gradient at the benchmarked 32K shape (14/2 heads, d =
     64, W = 1024, k = 16, needles; an 8-slot ring) and at 64K (a 4-slot ring:
     the selection lists take more LDS): the union kernel (64-key blocks
-    staged once per 48 queries) against bwd_dq_mfma (HBA_BWD_DQ_KERNEL=pair),
+    staged once per 32 queries) against bwd_dq_mfma (HBA_BWD_DQ_KERNEL=pair),
     which the oracle tests pin at small n.  Both compute the same sums in a
     different order and softmax form (fixed shift, its scale folded into the
     bf16 query operand, against a running max), so dq, and dk / dv through
