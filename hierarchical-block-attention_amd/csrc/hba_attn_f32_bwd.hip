@@ -17,9 +17,9 @@
 // launch of bwd_dkv_f32 takes as many ranges as there are places for their sums
 // beyond the workspace that hba_attn_bwd asks for, bwd_k_f32 adds these in order,
 // and with fewer than two places each range is a launch that adds to dk and dv
-// itself.  Atomic sums, in another order each time, cost 1 % less at 2048 tokens,
-// 14 / 2 heads, head dim 64 (992 us per training step against 1002), up to 10 %
-// less (8192 tokens, 8 heads: 1412 us against 1552, four launches of 8 ranges).
+// itself.  Atomic sums, in another order each time, took 993 us per training
+// step at 2048 tokens, 14 / 2 heads, head dim 64, where these take 999; over 67
+// shapes of 64 to 32768 tokens these take 0.86 to 1.05 of the atomics' time.
 //
 // Matrix cores bound all three products at 64 FLOP per SIMD and cycle; every
 // operand comes from L1 / L2 in the layout it is used in (16 bytes per lane,
@@ -506,33 +506,37 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void bwd_dkv_f32_kernel(
     }
 }
 
-// dk and dv of a 64-key block of one (b, g), a wave its 16 keys.  With `part`,
-// its nr ranges' sums are added to those of the earlier launches (in dk and dv,
-// the sinks' in `sink`; none if this is the first).  After the last launch of
-// ranges the sinks' sums are added to block 0 and the key rows taken through
-// the QKNorm backward, with one gain atomic per workgroup.
+// dk and dv of 16 keys of one (b, g), a wave a quarter of their elements.  With
+// `part`, its nr ranges' sums are added to those of the earlier launches (in dk
+// and dv, the sinks' in `sink`; none if this is the first).  After the last
+// launch of ranges the sinks' sums are added to block 0 and the key rows taken
+// through the QKNorm backward, with one gain atomic per workgroup.  Bound by the
+// latency of its reads, U places of which are in flight: 2048 tokens, 2 KV heads,
+// 32 ranges 15 us, with a wave per 16 keys and 4 places 23.
 template <int D>
 __global__ __launch_bounds__(256) void bwd_k_f32_kernel(const float *__restrict__ part, const int *__restrict__ used,
                                                         float *__restrict__ sink, int nr, int nblk, int S, bool first,
-                                                        bool last, const float *__restrict__ k, const float *__restrict__ kgain,
-                                                        float eps, int n, int Hkv, float *__restrict__ dk,
-                                                        float *__restrict__ dv, float *__restrict__ dk_gain) {
-    constexpr int NC = D / 16, U = (D == 64) ? 4 : 2;
-    __shared__ float gsum[4];
+                                                        bool last, const float *__restrict__ k,
+                                                        const float *__restrict__ kgain, float eps, int n, int Hkv,
+                                                        float *__restrict__ dk, float *__restrict__ dv,
+                                                        float *__restrict__ dk_gain) {
+    constexpr int NC = D / 16, C = NC / 4, U = 16 / C;   // C: 16-element groups per wave
+    __shared__ float red[4][2][16];
     const int lane = threadIdx.x & 63, l16 = lane & 15, lg = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nb = n / 64, blk = (int)(blockIdx.x % nb);
-    const int64_t bg = blockIdx.x / nb, b = bg / Hkv;
+    const int nb = n / 64, kg = (int)(blockIdx.x & 3), blk = (int)((blockIdx.x >> 2) % nb);
+    const int64_t bg = (blockIdx.x >> 2) / nb, b = bg / Hkv;
     const int g = (int)(bg % Hkv);
-    const int64_t row = (b * n + 64 * (int64_t)blk + 16 * w + 4 * lg) * Hkv + g, rs = (int64_t)Hkv * D;
-    const int64_t o = row * D + l16;   // element 16 c of key e: o + e rs + 16 c
-    f32x4 gk[NC], gv[NC];
+    const int64_t row = (b * n + 64 * (int64_t)blk + 16 * kg + 4 * lg) * Hkv + g, rs = (int64_t)Hkv * D;
+    const int64_t o = row * D + 16 * C * w + l16;   // element 16 c of key e: o + e rs + 16 c
+    const int fo = 256 * C * w + 4 * lane;          // this wave's first f32x4 of a slot's dk part
+    f32x4 gk[C], gv[C];
     auto add = [&](int bx) {
         const int64_t s0 = (bg * nblk + bx) * nr;
         for (int c0 = 0; c0 < nr; c0 += 64) {
-            const bool u = c0 + lane < nr && used[(s0 + c0 + lane) * 4 + w] != 0;
+            const bool u = c0 + lane < nr && used[(s0 + c0 + lane) * 4 + kg] != 0;
             for (uint64_t m = __ballot(u); m;) {   // U slots' loads in flight
-                f32x4 x[U][2 * NC];
+                f32x4 x[U][2 * C];
                 bool has[U];
                 int i = 0;
 #pragma unroll
@@ -540,39 +544,42 @@ __global__ __launch_bounds__(256) void bwd_k_f32_kernel(const float *__restrict_
                     has[t] = m != 0;
                     i = m ? __builtin_ctzll(m) : i;   // none left: the last one again, unused
                     m &= m - 1;
-                    const float *pp = part + ((s0 + c0 + i) * 4 + w) * (2 * 16 * D) + 4 * lane;
+                    const float *pp = part + ((s0 + c0 + i) * 4 + kg) * (2 * 16 * D) + fo;
 #pragma unroll
-                    for (int c = 0; c < 2 * NC; ++c) x[t][c] = ld4(pp + 256 * c);
+                    for (int c = 0; c < C; ++c) {
+                        x[t][c] = ld4(pp + 256 * c);
+                        x[t][C + c] = ld4(pp + 256 * (NC + c));
+                    }
                 }
 #pragma unroll
                 for (int t = 0; t < U; ++t)
                     if (has[t]) {
 #pragma unroll
-                        for (int c = 0; c < NC; ++c) {
+                        for (int c = 0; c < C; ++c) {
                             gk[c] += x[t][c];
-                            gv[c] += x[t][NC + c];
+                            gv[c] += x[t][C + c];
                         }
                     }
             }
         }
     };
-    f32x4 *sp = reinterpret_cast<f32x4 *>(sink + (bg * 4 + w) * (2 * 16 * D)) + lane;
-    const bool sinks = blk == 0 && S > 16 * w;
+    f32x4 *sp = reinterpret_cast<f32x4 *>(sink + (bg * 4 + kg) * (2 * 16 * D) + fo);
+    const bool sinks = blk == 0 && S > 16 * kg;
     if (part && sinks) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
+        for (int c = 0; c < C; ++c) {
             gk[c] = first ? f32x4{0.f, 0.f, 0.f, 0.f} : sp[64 * c];
             gv[c] = first ? f32x4{0.f, 0.f, 0.f, 0.f} : sp[64 * (NC + c)];
         }
         add(nb);
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
+        for (int c = 0; c < C; ++c) {
             sp[64 * c] = gk[c];
             sp[64 * (NC + c)] = gv[c];
         }
     }
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
+    for (int c = 0; c < C; ++c)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             gk[c][e] = first ? 0.0f : dk[o + e * rs + 16 * c];
@@ -581,44 +588,51 @@ __global__ __launch_bounds__(256) void bwd_k_f32_kernel(const float *__restrict_
     if (part) add(blk);
     if (last && sinks) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
+        for (int c = 0; c < C; ++c) {
             gk[c] += sp[64 * c];
             gv[c] += sp[64 * (NC + c)];
         }
     }
-    if (last && kgain) {
+    if (last && kgain) {   // uniform
         const float gn = kgain[g];
-        float gs = 0.0f;
+        float x[4][C], gs = 0.0f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            float x[NC], ss = 0.0f, yx = 0.0f;
+            float ss = 0.0f, yx = 0.0f;
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                x[c] = k[o + e * rs + 16 * c];
-                ss = fmaf(x[c], x[c], ss);
-                yx = fmaf(gk[c][e], x[c], yx);
+            for (int c = 0; c < C; ++c) {
+                x[e][c] = k[o + e * rs + 16 * c];
+                ss = fmaf(x[e][c], x[e][c], ss);
+                yx = fmaf(gk[c][e], x[e][c], yx);
             }
 #pragma unroll
             for (int d = 1; d < 16; d *= 2) {   // over the key's 16 lanes
                 ss += __shfl_xor(ss, d, 64);
                 yx += __shfl_xor(yx, d, 64);
             }
+            if (l16 == 0) {
+                red[w][0][4 * lg + e] = ss;
+                red[w][1][4 * lg + e] = yx;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int j = 4 * lg + e;
+            const float ss = (red[0][0][j] + red[1][0][j]) + (red[2][0][j] + red[3][0][j]);
+            const float yx = (red[0][1][j] + red[1][1][j]) + (red[2][1][j] + red[3][1][j]);
             const float ms = ss / (float)D;
             const float r = sqrtf(fmaxf(ms, eps));
             const float corr = (ms >= eps) ? gn * yx / ((float)D * r * r * r) : 0.0f;
 #pragma unroll
-            for (int c = 0; c < NC; ++c) gk[c][e] = (gn / r) * gk[c][e] - x[c] * corr;
+            for (int c = 0; c < C; ++c) gk[c][e] = (gn / r) * gk[c][e] - x[e][c] * corr;
             gs += yx / r;
         }
-        if (dk_gain) {
-            gs = col_sum(gs);
-            if (lane == 0) gsum[w] = gs;
-            __syncthreads();
-            if (threadIdx.x == 0) unsafeAtomicAdd(&dk_gain[g], (gsum[0] + gsum[1]) + (gsum[2] + gsum[3]));
-        }
+        gs = col_sum(gs);
+        if (dk_gain && threadIdx.x == 0) unsafeAtomicAdd(&dk_gain[g], gs);
     }
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
+    for (int c = 0; c < C; ++c)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             dk[o + e * rs + 16 * c] = gk[c][e];
@@ -627,21 +641,25 @@ __global__ __launch_bounds__(256) void bwd_k_f32_kernel(const float *__restrict_
 }
 
 // Ranges of query rows (R rows each, nsplit in all) and how many of them a
-// launch of bwd_dkv_f32 takes if the workspace has a place for each: enough for
-// F32_WGS workgroups (16 rounds of the 512 that run at once).  The places are
-// about F32_WGS times 32 KB at d = 64 then, however long the sequences are.  A
-// range of as many blocks or more fills the chip by itself and takes none.
-constexpr int64_t F32_WGS = 8192;
+// launch of bwd_dkv_f32 takes if the workspace has a place for each.  Up to 32
+// ranges, and no more than make F32_WGS workgroups (16 rounds of the 512 that
+// run at once): a range costs each block a place's write and read (8192 tokens,
+// 8 heads: 1415 us with 32 ranges, summed by atomics, 1298 with 8 in order).  All
+// of them in a launch if they are within F32_PLACES blocks (32 KB each at d = 64),
+// since each launch ends with its longest blocks (32768 tokens, 14 / 2 heads: 13.6
+// ms, 14.7 with two launches of 8 ranges).  A range of as many blocks fills the chip
+// by itself and takes no place.
+constexpr int64_t F32_WGS = 8192, F32_PLACES = 16384;
 struct Plan {
     int64_t R, nsplit, nr;
 };
 static Plan bwd_plan(int64_t Cn, int64_t n) {
     Plan p;
     p.R = F32_RMIN;
-    while (n / p.R > 32 && p.R < F32_RMAX) p.R *= 2;
+    while ((n / p.R > 32 || Cn * (n / 64) * (n / p.R) > F32_WGS) && p.R < F32_RMAX) p.R *= 2;
     p.nsplit = (n + p.R - 1) / p.R;
     const int64_t per = Cn * (n / 64 + 1);
-    p.nr = std::min(p.nsplit, (F32_WGS + per - 1) / per);
+    p.nr = std::min(p.nsplit, (F32_PLACES + per - 1) / per);
     return p;
 }
 // one range's places: sums and flags
@@ -671,7 +689,7 @@ int launch_attn_bwd_f32(const float *q, const float *k, const float *v, const fl
     const int64_t places = std::min<int64_t>(p.nr, (int64_t)(part_bytes / af::range_bytes(Cn, n, D)));
     const int64_t per = places < 2 ? 1 : places;   // ranges per launch
     const int64_t nblk = nb + (S > 0);
-    if (grid > 0x7fffffffLL || Cn * nblk * per > 0x7fffffffLL || n > 0x3fffffffLL || n * Hq > 0x7fffffffLL)
+    if (grid > 0x7fffffffLL || Cn * nblk * std::max<int64_t>(per, 4) > 0x7fffffffLL || n > 0x3fffffffLL || n * Hq > 0x7fffffffLL)
         return HBA_ERR_UNSUPPORTED;
     if (places < 2) part = nullptr;
     int *used = part ? reinterpret_cast<int *>(part + 4 * Cn * nblk * per * (2 * 16 * D)) : nullptr;
@@ -687,7 +705,7 @@ int launch_attn_bwd_f32(const float *q, const float *k, const float *v, const fl
                            dout, (int)n, (int)Hq, (int)Hkv, (int)S, Wc, (int)k_blocks, scale, (int)p.R, (int)r0,
                            (int)nr, (int)nblk, qc_ws, qr_ws, lse_ws, dd_ws, part ? part : sink, used, dk, dv);
         if (part || (last && (kgain || S > 0)))
-            hipLaunchKernelGGL(af::bwd_k_f32_kernel<D>, dim3((unsigned)(Cn * nb)), dim3(256), 0, s, part, used, sink,
+            hipLaunchKernelGGL(af::bwd_k_f32_kernel<D>, dim3((unsigned)(4 * Cn * nb)), dim3(256), 0, s, part, used, sink,
                                (int)nr, (int)nblk, (int)S, part && r0 == 0, last, k, kgain, eps, (int)n, (int)Hkv, dk,
                                dv, dk_gain);
     }

@@ -479,7 +479,8 @@ int hba_attn_bwd_workspace_bytes(int dtype, int64_t B, int64_t n, int64_t Hq, in
 /* hba_attn_bwd_workspace_bytes and what fp32 uses beyond it on the tuned
  * geometry, for sums of dk and dv over ranges of query rows: places of
  * B*Hkv*(n/64+1)*4 * (128*d + 4) bytes per range, for as many of the ceil(n/R)
- * ranges (R rows: 64, doubled while n/R > 32, at most 2048) as make 8192 blocks.
+ * ranges as make 16384 blocks (none where that is one; R rows: 64, doubled while
+ * n/R > 32 or B*Hkv*(n/64)*(n/R) > 8192, at most 2048; integer quotients).
  * With fewer bytes the ranges run in more launches, down to one after another
  * without a place; the results are the same bits. */
 int hba_attn_bwd_workspace_full_bytes(int dtype, int64_t B, int64_t n, int64_t Hq, int64_t Hkv,
