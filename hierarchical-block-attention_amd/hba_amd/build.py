@@ -81,7 +81,8 @@ def _compile(src):
         r = subprocess.run([HIPCC, *FLAGS, "-save-temps=obj", "-c", src, "-o", out], capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"hipcc failed on {src}:\n{r.stderr}")
-        with open(os.path.join(tmp, f"{name}-hip-amdgcn-amd-amdhsa-{ARCH}.s")) as f:
+        asm, = glob.glob(os.path.join(tmp, f"{name}-hip-*{ARCH}.s"))
+        with open(asm) as f:
             lost = lost_spills(f.read())
         if lost:
             raise RuntimeError(f"{src}: the compiler placed vector instructions before an exec restore, where not "

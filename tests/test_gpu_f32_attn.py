@@ -250,9 +250,9 @@ def _c_bwd(t, kc, kr, cos, sin, out, shape, nbytes=None):
         nbytes = b.value
     g = [torch.full((x.numel() + 8,), math.nan, dtype=x.dtype, device=dev)
          [x.data_ptr() % 16 // x.element_size():][:x.numel()].view(x.shape) for x in t[:3]]
-    gg = [torch.zeros_like(x) for x in (t[3], t[4])]
+    gg = [torch.zeros(h, device=dev) for h in (Hq, Hkv)]
     ws = torch.full((nbytes,), 255, dtype=torch.uint8, device=dev)
-    p = lambda x: x.data_ptr()
+    p = lambda x: None if x is None else x.data_ptr()
     st = lib.hba_attn_bwd(dt, p(t[0]), p(t[1]), p(t[2]), p(kc), p(kr), p(t[3]), p(t[4]), 1e-6, p(cos), p(sin), p(t[5]),
                           p(t[6]), p(out), p(t[7]), t[0].shape[0], n, Hq, Hkv, d, S, W, 64, k, 0.125, p(ws), nbytes,
                           *(p(x) for x in g + gg), torch.cuda.current_stream().cuda_stream)
@@ -260,7 +260,7 @@ def _c_bwd(t, kc, kr, cos, sin, out, shape, nbytes=None):
     return g
 
 
-def _bwd_args(shape, dev, dt=torch.float32):
+def _bwd_args(shape, dev, dt=torch.float32, gains=True):
     n, Hq, Hkv, d, S, W, k = shape
     q, kx, v, gq, gk, idx, cnt = (x[:1] if x.dim() > 1 else x for x in _inputs(*shape))
     q, kx, v = (x.to(dt) for x in (q, kx, v))
@@ -268,6 +268,8 @@ def _bwd_args(shape, dev, dt=torch.float32):
     dout = torch.randn(q.shape, generator=torch.Generator().manual_seed(5)).to(dt)
     cos, sin = hba_amd.rope_tables(n, d, 10000.0, dev)
     t = [x.to(dev) for x in (q, kx, v, gq, gk, idx, cnt, dout)]
+    if not gains:
+        t[3] = t[4] = None
     kc, kr, vt = ops.prep_keys(t[1], t[2], t[4], 1e-6, cos, sin)
     out = ops.attn_fwd(t[0], t[3], t[4], 1e-6, kc, kr, vt, cos, sin, t[5], t[6], S, W, 0.125)
     return t, kc, kr, cos, sin, out
@@ -286,13 +288,14 @@ def test_backward_of_long_ranges_against_the_generic_kernels():
 
 
 #                                    n     Hq Hkv d   S   W    k
+@pytest.mark.parametrize("gains", [True, False])
 @pytest.mark.parametrize("shape", [(2112, 6, 2, 64, 20, 130, 3), (832, 2, 1, 128, 4, 1000, 5), (192, 7, 1, 64, 0, 64, 3)])
-def test_backward_is_the_same_bits_from_run_to_run_and_with_any_workspace(shape):
-    """dq, dk and dv of two runs, and of a workspace with places for no, for
-    three and for all ranges of query rows."""
+def test_backward_is_the_same_bits_from_run_to_run_and_with_any_workspace(shape, gains, monkeypatch):
+    """dq, dk and dv of two runs, of a workspace with places for no, for three
+    and for all ranges of query rows, and of the op when memory is out."""
     n, Hq, Hkv, d, S, W, k = shape
     dev = torch.device("cuda")
-    t, kc, kr, cos, sin, out = _bwd_args(shape, dev)
+    t, kc, kr, cos, sin, out = _bwd_args(shape, dev, gains=gains)
     lib, ws = _lib.lib(), {}
     for name in ("bytes", "full_bytes"):
         b = ctypes.c_size_t(0)
@@ -301,8 +304,21 @@ def test_backward_is_the_same_bits_from_run_to_run_and_with_any_workspace(shape)
     place = Hkv * (n // 64 + 1) * 4 * (128 * d + 4)
     assert ws["full_bytes"] - ws["bytes"] == -(-n // (128 if n > 2048 else 64)) * place
 
-    want = ops.attn_bwd(t[0], t[1], t[2], kc, kr, t[3], t[4], 1e-6, cos, sin, t[5], t[6], out, t[7], S, W, 0.125)[:3]
+    op = lambda: ops.attn_bwd(t[0], t[1], t[2], kc, kr, t[3], t[4], 1e-6, cos, sin, t[5], t[6], out, t[7], S, W, 0.125)[:3]
+    want = op()
     assert all(x.isfinite().all() for x in want)
+    empty, asked = torch.empty, []
+
+    def out_of_memory(*a, **kw):
+        if kw.get("dtype") == torch.uint8:
+            asked.append(a[0])
+            if a[0] == ws["full_bytes"]:
+                raise torch.OutOfMemoryError("no room")
+        return empty(*a, **kw)
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", out_of_memory)
+        assert all(torch.equal(a, b) for a, b in zip(op(), want))
+    assert asked == [ws["full_bytes"], ws["bytes"]]
     for nbytes in (ws["full_bytes"], ws["full_bytes"], ws["bytes"] + 3 * place + 64, ws["bytes"]):
         for name, a, b in zip(("dq", "dk", "dv"), _c_bwd(t, kc, kr, cos, sin, out, shape, nbytes), want):
             assert torch.equal(a, b), (name, nbytes)
